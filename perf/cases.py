@@ -1,0 +1,545 @@
+"""The work a user of this framework has it do, as cases that can be timed and checked.
+
+Every case goes through the public entry points of ``wavebem_amd.bem.BEMProblem``.  The
+meshes are the closed Wigley half-tank of ``wavebem_amd.mesh`` with a free surface displaced
+by a wave (the geometry a free-surface solver hands over at every step), and for the
+unstructured path a box beside a patch whose blocks meet at a valence-3 vertex.
+
+Kinds of pass:
+
+* ``step``      assemble_system + solve_system on device vectors: one BEM step;
+* ``moving``    set_support_points + assemble_system + solve_system on host vectors: what a
+                time loop's residual does for every state;
+* ``matrices``  assemble_system, the solid angles, one vmult and one compute_rhs on a partly
+                unstructured mesh;
+* ``product``   one constrained operator product on an assembled problem;
+* ``multi``     several right-hand sides solved together on an assembled problem;
+* ``adjoint``   transposed solve and the backward of the assembly (gradient of a drag);
+* ``tangent``   the Jacobian-vector product of a Newton step: frozen right-hand side, tangent
+                of the assembly, one solve;
+* ``gradients`` L2 projections of the normals and of the complete potential gradient.
+"""
+from __future__ import annotations
+
+import dataclasses
+import functools
+import math
+
+import numpy as np
+import torch
+
+from wavebem_amd import mesh as M
+from wavebem_amd.adjoint import hull_drag
+from wavebem_amd.bem import BEMProblem, Config
+
+TANK = ("nh", "nt", "nu", "nd", "ny", "nzd")
+
+
+def _tank(nh, nt, nu, nd, ny, nzd):
+    return dict(mesh="tank", nh=nh, nt=nt, nu=nu, nd=nd, ny=ny, nzd=nzd)
+
+
+def listed():
+    return [
+        # the headline step at 41,207 dofs, refinement around reduced-precision inner solves
+        dict(name="step_fp32ir_40k", kind="step", precision="fp32_ir",
+             **_tank(100, 22, 40, 56, 60, 10)),
+        # the same step in plain FP64
+        dict(name="step_fp64_40k", kind="step", precision="fp64",
+             **_tank(100, 22, 40, 56, 60, 10)),
+        # the residual evaluation of a time loop at 21,157 dofs, host vectors
+        dict(name="moving_fp32ir_20k", kind="moving", precision="fp32_ir",
+             **_tank(70, 16, 28, 40, 42, 8)),
+        # the small FP64 configuration (2,915 dofs)
+        dict(name="step_fp64_2.5k", kind="step", precision="fp64",
+             **_tank(24, 6, 10, 14, 14, 4)),
+        # the smallest step: launches and host work weigh most
+        dict(name="step_fp32ir_1k", kind="step", precision="fp32_ir",
+             **_tank(12, 4, 6, 8, 8, 3)),
+        # eight boundary-data sets solved together at 61,111 dofs
+        dict(name="multi8_fp32ir_60k", kind="multi", precision="fp32_ir", k=8,
+             **_tank(120, 28, 50, 70, 72, 12)),
+        # drag gradient at 10,951 dofs: transposed solve and backward of the assembly
+        dict(name="adjoint_fp64_10k", kind="adjoint", precision="fp64",
+             **_tank(48, 12, 20, 28, 30, 6)),
+        # one Newton Jacobian-vector product at 41,207 dofs
+        dict(name="tangent_fp32ir_40k", kind="tangent", precision="fp32_ir",
+             **_tank(100, 22, 40, 56, 60, 10)),
+        # partly unstructured mesh with a five-point rule, FP64
+        dict(name="matrices_fp64_mixed", kind="matrices", precision="fp64", mesh="mixed",
+             box=20, block=33, q=5),
+        # one operator product of a caller's own Krylov loop: the smallest call
+        dict(name="product_fp64_1k", kind="product", precision="fp64", **_tank(12, 4, 6, 8, 8, 3)),
+        # boundary-data and pressure projections at 10,951 dofs
+        dict(name="gradients_10k", kind="gradients", precision="fp32_ir",
+             **_tank(48, 12, 20, 28, 30, 6)),
+    ]
+
+
+# dof count of the base tank whose side counts draw() scales
+_BASE = dict(nh=48, nt=12, nu=20, nd=28, ny=30, nzd=6)
+_BASE_N = 10951
+
+
+def draw(rng):
+    kind = rng.choice(["step", "step", "moving", "matrices", "product", "multi", "adjoint",
+                       "tangent", "gradients"])
+    precision = rng.choice(["fp64", "fp32_ir"])
+    lo, hi = {"multi": (800, 30000), "adjoint": (600, 16000), "matrices": (700, 16000)}.get(
+        kind, (600, 40000))
+    n = math.exp(rng.uniform(math.log(lo), math.log(hi)))
+    if kind == "matrices":
+        # 6 (b + 1)^2 dofs of the box and about 3 m^2 of the patch
+        share = rng.uniform(0.2, 0.8)
+        return dict(kind=kind, precision=precision, mesh="mixed",
+                    box=max(3, round(math.sqrt(share * n / 6)) - 1),
+                    block=max(3, round(math.sqrt((1 - share) * n / 3))),
+                    q=rng.choice([3, 4, 4, 5]))
+    f = math.sqrt(n / _BASE_N)
+    c = dict(kind=kind, precision=precision, mesh="tank")
+    for key, least in zip(TANK, (6, 2, 3, 4, 4, 2)):
+        c[key] = max(least, round(_BASE[key] * f * rng.uniform(0.85, 1.1)))
+    if kind == "multi":
+        c["k"] = rng.choice([2, 3, 5, 8])
+    return c
+
+
+# ---------------------------------------------------------------- inputs
+@functools.lru_cache(maxsize=None)
+def _flat_tank(*sides):
+    return M.wigley_tank(**dict(zip(TANK, sides)))
+
+
+@functools.lru_cache(maxsize=None)
+def _mixed(box, block):
+    return M.merge_meshes(M.box_mesh(n=box),
+                          M.tri_block_mesh(n=block, centre=(3.0, 0.0, 0.0)))
+
+
+def _waves(X, rng, amplitude=2e-3):
+    """Points of z = 0 raised by a travelling wave of x and y (coincident dofs alike)."""
+    Y = X.copy()
+    top = Y[:, 2] == 0.0
+    p, q = rng.uniform(0.0, 2.0 * math.pi, 2)
+    x, y = Y[top, 0], Y[top, 1]
+    Y[top, 2] = amplitude * (np.cos(9.0 * x - p) + 0.5 * np.cos(7.0 * x + 5.0 * y - q))
+    return Y
+
+
+def _setup(case, seed):
+    """(mesh at rest, displaced support points, boundary data, hull speed, generator)."""
+    rng = np.random.default_rng(seed)
+    if case["mesh"] == "mixed":
+        m = _mixed(case["box"], case["block"])
+        X = m.support_points * (1.0 + 0.05 * rng.uniform(-1.0, 1.0, 3))
+        return m, X, rng.standard_normal(m.n_dofs), 0.0, rng
+    m = _flat_tank(*(case[k] for k in TANK))
+    bc, speed = M.wigley_bc(m, seed=seed)
+    return m, _waves(m.support_points, rng), bc, speed, rng
+
+
+def _config(case):
+    return Config(precision=case["precision"], solver_max_steps=5000,
+                  quadrature_order=case.get("q", 4))
+
+
+def _known(mesh, bc):
+    return bc * mesh.surface_nodes, bc * mesh.other_nodes
+
+
+def prepare(case, seed):
+    m, X, bc, speed, rng = _setup(case, seed)
+    kind = case["kind"]
+    moved = dataclasses.replace(m, support_points=X)
+    p = BEMProblem(m if kind == "moving" else moved, _config(case))
+    s = dict(kind=kind, p=p, X=X, bc=bc)
+    phi, dphi = _known(m, bc)
+    if kind not in ("matrices", "gradients"):
+        p.compute_constraints(bc)
+    if kind == "step":
+        s.update({k: torch.tensor(v, dtype=torch.float64, device="cuda")
+                  for k, v in (("bc", bc), ("phi", phi), ("dphi", dphi))})
+        torch.cuda.synchronize()
+    elif kind == "moving":
+        s.update(phi=phi, dphi=dphi)
+    elif kind == "matrices":
+        s.update(src=rng.standard_normal(m.n_dofs))
+    elif kind == "gradients":
+        s.update(phi=rng.standard_normal(m.n_dofs), dphi=rng.standard_normal(m.n_dofs))
+    elif kind == "product":
+        p.assemble_system()
+        s.update(src=rng.standard_normal(m.n_dofs))
+    elif kind == "multi":
+        tmp = np.stack([bc] + [M.wigley_bc(m, seed=seed + 1000 * v)[0]
+                               for v in range(1, case["k"])])
+        p.assemble_system()
+        s.update(tmp=tmp, phi=tmp * m.surface_nodes, dphi=tmp * m.other_nodes)
+    else:
+        p.assemble_system()
+        p.solve_system(phi, dphi, bc)
+        s.update(phi=phi, dphi=dphi)
+        if kind == "adjoint":
+            s["g"] = _drag_gradient(moved, phi, dphi, speed)
+        else:
+            s.update(_direction(m, X, rng))
+    return s
+
+
+def _drag_gradient(mesh, phi, dphi, speed):
+    """dJ/du of the hull drag: what an adjoint solve is called with."""
+    hull = mesh.cell_material == M.HULL
+    a = torch.tensor(phi, requires_grad=True)
+    b = torch.tensor(dphi, requires_grad=True)
+    J = hull_drag(torch.tensor(mesh.support_points), mesh.cell_dofs[hull],
+                  mesh.cell_orient[hull], a, b, torch.zeros(mesh.n_dofs, dtype=torch.float64),
+                  speed)
+    ga, gb = torch.autograd.grad(J, (a, b))
+    return ga.numpy() * mesh.other_nodes + gb.numpy() * mesh.surface_nodes
+
+
+def _direction(mesh, X, rng):
+    """A Newton direction: free-surface elevations dx (z only) and potentials v."""
+    a, b = rng.standard_normal(2), rng.uniform(0.0, 2.0 * math.pi, 2)
+    top = mesh.support_points[:, 2] == 0.0
+    dx = np.zeros_like(X)
+    dx[top, 2] = 1e-3 * (a[0] * np.sin(11.0 * X[top, 0] + b[0]) + np.cos(6.0 * X[top, 1]))
+    v = 1e-3 * (a[1] * np.cos(8.0 * X[:, 0] - b[1]) + np.sin(5.0 * X[:, 1]))
+    return dict(dx=dx, v=v * mesh.surface_nodes)
+
+
+# ---------------------------------------------------------------- one pass
+def run(s):
+    p, kind = s["p"], s["kind"]
+    if kind == "step":
+        p.assemble_system()
+        p.solve_system_dev(s["phi"].data_ptr(), s["dphi"].data_ptr(), s["bc"].data_ptr())
+        return dict(phi=s["phi"], dphi=s["dphi"])
+    if kind == "moving":
+        p.set_support_points(s["X"])
+        p.assemble_system()
+        p.solve_system(s["phi"], s["dphi"], s["bc"])
+        return dict(phi=s["phi"], dphi=s["dphi"])
+    if kind == "matrices":
+        p.assemble_system()
+        return dict(alpha=p.compute_alpha(), vmult=p.vmult(s["src"]), rhs=p.compute_rhs(s["src"]))
+    if kind == "product":
+        return dict(dst=p.constrained_vmult(s["src"]))
+    if kind == "multi":
+        p.solve_system_multi(s["phi"], s["dphi"], s["tmp"])
+        return dict(phi=s["phi"], dphi=s["dphi"])
+    if kind == "adjoint":
+        lam = p.solve_adjoint(s["g"])
+        return dict(lam=lam, grad=p.residual_vjp(lam, s["phi"], s["dphi"]))
+    if kind == "tangent":
+        b = -p.residual(s["v"], np.zeros(p.n))
+        b -= p.residual_jvp(s["dx"], s["phi"], s["dphi"])
+        return dict(b=b, du=p.solve_rhs(b))
+    return dict(normals=p.compute_normals(),
+                grads=p.compute_potential_gradients(s["phi"], s["dphi"]))
+
+
+# ---------------------------------------------------------------- work and tolerances
+def _sizes(case):
+    if case["mesh"] == "mixed":
+        m = _mixed(case["box"], case["block"])
+    else:
+        m = _flat_tank(*(case[k] for k in TANK))
+    return m.n_dofs, m.n_cells, case.get("q", 4) ** 2
+
+
+def work(case):
+    """Assembly: 36 flops per (row, quadrature point), G and H written once (16 bytes per
+    entry pair in FP64, 12 as FP32 + bf16).  A solve or a product cannot do without one read
+    of the selected operator, a right-hand side without one of the other columns (8 or 6
+    bytes and 2 flops per entry); a tangent or a backward of the assembly evaluates every
+    (row, point) again, with about twice the flops."""
+    n, nc, nq = _sizes(case)
+    e = 8 if case["precision"] == "fp64" else 6
+    kind, n2 = case["kind"], float(n) * n
+    ev = 36.0 * n * nc * nq
+    mesh = 8.0 * 3 * n + 17.0 * nc
+    if kind in ("step", "moving", "matrices"):
+        return {"bytes": (2 + 2) * e * n2 + mesh + 48.0 * n, "flops": ev + 4 * n2}
+    if kind == "product":
+        return {"bytes": e * n2 + 16.0 * n, "flops": 2 * n2}
+    if kind == "multi":
+        return {"bytes": 2 * e * n2 + 24.0 * n * case["k"], "flops": 4 * n2 * case["k"]}
+    if kind == "adjoint":
+        return {"bytes": e * n2 + mesh + 72.0 * n, "flops": 2 * n2 + 2 * ev}
+    if kind == "tangent":
+        return {"bytes": 2 * e * n2 + mesh + 72.0 * n, "flops": 4 * n2 + 2 * ev}
+    # a 4x4 mass block and six right-hand sides per cell, 9 entries per row and field
+    return {"bytes": mesh + 64.0 * n, "flops": 2.0 * nc * nq * 150}
+
+
+def tolerance(case):
+    """About four times the largest distances seen from ``exact``.  Solutions: GMRES stops at
+    an absolute preconditioned residual of 1e-10 against data of 1e-3, which leaves them
+    6.6e-10 off (2.9k dofs), the gradient of the adjoint 1.6e-9 (11k).  Products: sums of
+    FP64 products 7e-14, FP32 + bf16 storage (2^-33 per entry) 3.5e-12.  Projections: CG to
+    1e-14 per field, 2.6e-14."""
+    if case["kind"] in ("step", "moving", "multi", "tangent"):
+        return {"rel": 1e-8}
+    if case["kind"] == "adjoint":
+        return {"rel": 3e-8}
+    if case["kind"] in ("matrices", "product"):
+        return {"rel": 1e-12 if case["precision"] == "fp64" else 1e-10}
+    return {"rel": 1e-12}
+
+
+# ---------------------------------------------------------------- the same in plain torch
+def _gauss01(q):
+    t, w = np.polynomial.legendre.leggauss(q)
+    return 0.5 * (t + 1.0), 0.5 * w
+
+
+def _regular_rule(q):
+    t, w = _gauss01(q)
+    return np.tile(t, q), np.repeat(t, q), np.tile(w, q) * np.repeat(w, q)
+
+
+def _singular_rule(s, vertex):
+    """The polar rule for a 1/R singularity at a vertex of the unit square: two triangles,
+    Gauss in the radial coordinate and in the tangent of the angle."""
+    u, v, w = _regular_rule(s)
+    a, b = u, u * np.tan(0.25 * math.pi * v)
+    ww = w * 0.25 * math.pi / np.cos(0.25 * math.pi * v) * np.hypot(a, b)
+    x, y = np.concatenate([a, b]), np.concatenate([b, a])
+    w = np.concatenate([ww, ww])
+    x, y = {0: (x, y), 1: (1 - y, x), 2: (y, 1 - x), 3: (1 - x, 1 - y)}[vertex]
+    return x, y, w
+
+
+def _shape(x, y):
+    f = np.stack([(1 - x) * (1 - y), x * (1 - y), (1 - x) * y, x * y], 1)
+    fx = np.stack([-(1 - y), 1 - y, -y, y], 1)
+    fy = np.stack([-(1 - x), -x, 1 - x, x], 1)
+    return [torch.tensor(a, device="cuda") for a in (f, fx, fy)]
+
+
+class _Reference:
+    """Collocation BEM of one mesh in plain torch, 64 bits, on the GPU."""
+
+    def __init__(self, mesh, X, q=4, s=5):
+        dev = "cuda"
+        self.cells = torch.tensor(mesh.cell_dofs, dtype=torch.long, device=dev)
+        self.sign = torch.tensor(mesh.cell_orient, dtype=torch.float64, device=dev)
+        self.surf = torch.tensor(mesh.surface_nodes, dtype=torch.float64, device=dev)
+        self.X = torch.tensor(X, dtype=torch.float64, device=dev)
+        self.n, self.nc = mesh.n_dofs, mesh.n_cells
+        rx, ry, rw = _regular_rule(q)
+        self.rule = (*_shape(rx, ry), torch.tensor(rw, device=dev))
+        self.srule = []
+        for v in range(4):
+            sx, sy, sw = _singular_rule(s, v)
+            self.srule.append((*_shape(sx, sy), torch.tensor(sw, device=dev)))
+        # coincident dofs, and per row the cells that hold one of its class (first vertex)
+        _, cls = np.unique(np.round(X, 9) + 0.0, axis=0, return_inverse=True)
+        cls = np.asarray(cls).reshape(-1)
+        self.cls = cls
+        members = [[] for _ in range(cls.max() + 1)]
+        for d, k in enumerate(cls):
+            members[k].append(d)
+        self.members = members
+        touch = [dict() for _ in members]
+        for c, vs in enumerate(np.asarray(mesh.cell_dofs)):
+            for k in range(4):
+                touch[cls[vs[k]]].setdefault(c, k)
+        pr = [(d, c, k) for d in range(self.n) for c, k in touch[cls[d]].items()]
+        pr = torch.tensor(pr, dtype=torch.long, device=dev)
+        self.pr, self.pc, self.pv = pr[:, 0], pr[:, 1], pr[:, 2]
+
+    def geometry(self, X, cells, sign, rule):
+        """Points, normals times JxW and JxW of ``rule`` on the given cells."""
+        f, fx, fy, w = rule
+        V = X[cells]
+        y, a, b = f @ V, fx @ V, fy @ V
+        N = torch.linalg.cross(a, b) * (w[:, None] * sign[:, None, None])
+        return y, N, torch.sqrt((N * N).sum(2))
+
+    @staticmethod
+    def kernels(y, N, J, x):
+        """(single, double): JxW / 4 pi r and (x - y).N / 4 pi r^3."""
+        R = y - x
+        ri = torch.rsqrt((R * R).sum(-1))
+        return J * ri / (4 * math.pi), -(R * N).sum(-1) * ri ** 3 / (4 * math.pi)
+
+    def chunks(self):
+        step = max(1, int(3e7 // (self.nc * self.rule[3].numel())))
+        return [(a, min(self.n, a + step)) for a in range(0, self.n, step)]
+
+    def matrices(self):
+        G = torch.zeros(self.n, self.n, dtype=torch.float64, device="cuda")
+        H = torch.zeros_like(G)
+        y, N, J = self.geometry(self.X, self.cells, self.sign, self.rule)
+        flat = self.cells.reshape(-1)
+        for a, b in self.chunks():
+            g, h = self.kernels(y[None], N[None], J[None], self.X[a:b, None, None])
+            in_ = (self.pr >= a) & (self.pr < b)
+            for t, out in ((g, G), (h, H)):
+                t = t @ self.rule[0]
+                t[self.pr[in_] - a, self.pc[in_]] = 0.0
+                out[a:b].index_add_(1, flat, t.reshape(b - a, -1))
+        for v in range(4):
+            k = self.pv == v
+            r, c = self.pr[k], self.pc[k]
+            y, N, J = self.geometry(self.X, self.cells[c], self.sign[c], self.srule[v])
+            g, h = self.kernels(y, N, J, self.X[r][:, None])
+            at = (r[:, None].expand(-1, 4), self.cells[c])
+            G.index_put_(at, g @ self.srule[v][0], accumulate=True)
+            H.index_put_(at, h @ self.srule[v][0], accumulate=True)
+        return G, H
+
+    def residual_rows(self, X, phi, psi, a, b):
+        """Rows a .. b - 1 of sum_j H_ij (phi_j - phi_i) - G_ij psi_j."""
+        y, N, J = self.geometry(X, self.cells, self.sign, self.rule)
+        f = self.rule[0]
+        g, h = self.kernels(y[None], N[None], J[None], X[a:b, None, None])
+        t = (h * ((phi[self.cells] @ f.T)[None] - phi[a:b, None, None])
+             - g * (psi[self.cells] @ f.T)[None]).sum(2)
+        keep = torch.ones(b - a, self.nc, dtype=torch.float64, device="cuda")
+        in_ = (self.pr >= a) & (self.pr < b)
+        keep[self.pr[in_] - a, self.pc[in_]] = 0.0
+        return (t * keep).sum(1)
+
+    def residual_singular(self, X, phi, psi):
+        out = 0.0
+        for v in range(4):
+            k = self.pv == v
+            r, c = self.pr[k], self.pc[k]
+            f = self.srule[v][0]
+            y, N, J = self.geometry(X, self.cells[c], self.sign[c], self.srule[v])
+            g, h = self.kernels(y, N, J, X[r][:, None])
+            t = (h * (phi[self.cells[c]] @ f.T - phi[r][:, None])
+                 - g * (psi[self.cells[c]] @ f.T)).sum(1)
+            out = out + torch.zeros(self.n, dtype=torch.float64,
+                                    device="cuda").index_add(0, r, t)
+        return out
+
+    def constraints(self, tmp):
+        """(row, other dof or -1, inhomogeneity) of the double-node rules (at most one
+        Dirichlet dof per set here): Neumann dofs beside a Dirichlet one take its value,
+        the rest of a Neumann set equals its first dof."""
+        out = []
+        surf = self.surf.cpu().numpy()
+        for ds in self.members:
+            d = [i for i in ds if surf[i] == 1.0]
+            first = d[0] if d else ds[0]
+            for k in ds:
+                if k != first:
+                    out.append((k, -1, tmp[first]) if d else (k, first, 0.0))
+        return out
+
+    def system(self, G, H, tmp):
+        """Constrained operator and right-hand side(s) for boundary data tmp (n,) or (n, k)."""
+        S, O = self.surf, 1.0 - self.surf
+        alpha = -H.sum(1)
+        A = H * O - G * S
+        A.diagonal().add_(alpha * O)
+        t = torch.tensor(np.asarray(tmp), dtype=torch.float64, device="cuda").reshape(self.n, -1)
+        b = -H @ (S[:, None] * t) - (alpha * S)[:, None] * t + G @ (O[:, None] * t)
+        self.rows = []
+        for k in range(t.shape[1]):
+            for row, col, inhom in self.constraints(t[:, k].cpu().numpy()):
+                if k == 0:
+                    self.rows.append(row)
+                    A[row] = 0.0
+                    A[row, row] = 1.0
+                    if col >= 0:
+                        A[row, col] = -1.0
+                b[row, k] = inhom
+        return A, b
+
+    def projections(self, phi, psi):
+        """Unit nodal normals and the complete potential gradient, mean over coincident dofs."""
+        f, fx, fy, w = self.rule
+        V = self.X[self.cells]
+        a, b = fx @ V, fy @ V
+        cr = torch.linalg.cross(a, b)
+        J = cr.norm(dim=2)
+        nrm = cr / J[:, :, None] * self.sign[:, None, None]
+        J = J * w
+        g00, g01, g11 = (a * a).sum(2), (a * b).sum(2), (b * b).sum(2)
+        det = g00 * g11 - g01 * g01
+        ux, uy = phi[self.cells] @ fx.T, phi[self.cells] @ fy.T
+        grad = (((g11 * ux - g01 * uy) / det)[..., None] * a
+                + ((g00 * uy - g01 * ux) / det)[..., None] * b
+                + nrm * (psi[self.cells] @ f.T)[..., None])
+        mass = torch.zeros(self.n, self.n, dtype=torch.float64, device="cuda")
+        blocks = (f.T[None] * J[:, None, :]) @ f
+        mass.index_put_((self.cells[:, :, None].expand(-1, 4, 4),
+                         self.cells[:, None, :].expand(-1, 4, 4)), blocks, accumulate=True)
+        rhs = torch.zeros(self.n, 6, dtype=torch.float64, device="cuda")
+        e = (f.T[None] * J[:, None, :]) @ torch.cat([nrm, grad], 2)
+        rhs.index_add_(0, self.cells.reshape(-1), e.reshape(-1, 6))
+        x = torch.linalg.solve(mass, rhs)
+        nn = x[:, :3] / x[:, :3].norm(dim=1, keepdim=True)
+        g = x[:, 3:].cpu().numpy()
+        out = g.copy()
+        for ds in self.members:
+            out[ds] = g[ds].mean(0)
+        return nn.cpu().numpy(), out
+
+
+_EXACT_MOST = 11500  # dofs up to which the dense 64-bit system is formed
+
+
+def exact(case, seed):
+    m, X, bc, speed, rng = _setup(case, seed)
+    if m.n_dofs > _EXACT_MOST:
+        return None
+    ref = _Reference(m, X, q=case.get("q", 4))
+    kind = case["kind"]
+
+    def gpu(a):
+        return torch.tensor(a, dtype=torch.float64, device="cuda")
+
+    if kind == "gradients":
+        phi, psi = rng.standard_normal(m.n_dofs), rng.standard_normal(m.n_dofs)
+        nn, g = ref.projections(gpu(phi), gpu(psi))
+        return dict(normals=nn, grads=g)
+    G, H = ref.matrices()
+    if kind == "matrices":
+        src = gpu(rng.standard_normal(m.n_dofs))
+        S, O, alpha = ref.surf, 1.0 - ref.surf, -H.sum(1)
+        return dict(alpha=alpha, vmult=H @ (O * src) - G @ (S * src) + alpha * O * src,
+                    rhs=G @ (O * src) - H @ (S * src) - alpha * S * src)
+    if kind == "multi":
+        tmp = np.stack([bc] + [M.wigley_bc(m, seed=seed + 1000 * v)[0]
+                               for v in range(1, case["k"])])
+        A, b = ref.system(G, H, tmp.T)
+        x = torch.linalg.solve(A, b).T.cpu().numpy()
+        S = m.surface_nodes
+        return dict(phi=S * tmp + (1 - S) * x, dphi=(1 - S) * tmp + S * x)
+    A, b = ref.system(G, H, bc)
+    if kind == "product":
+        return dict(dst=A @ gpu(rng.standard_normal(m.n_dofs)))
+    x = torch.linalg.solve(A, b)[:, 0]
+    S = ref.surf
+    t = gpu(bc)
+    phi, psi = S * t + (1 - S) * x, (1 - S) * t + S * x
+    if kind in ("step", "moving"):
+        return dict(phi=phi, dphi=psi)
+    Xg = ref.X
+    if kind == "adjoint":
+        moved = dataclasses.replace(m, support_points=X)
+        g = _drag_gradient(moved, phi.cpu().numpy(), psi.cpu().numpy(), speed)
+        lam = torch.linalg.solve(A.T, gpu(g))
+        w = lam.clone()
+        w[ref.rows] = 0.0
+        Xr = Xg.clone().requires_grad_(True)
+        grad = torch.autograd.grad(w @ ref.residual_singular(Xr, phi, psi), Xr)[0]
+        for a, e in ref.chunks():
+            v = w[a:e] @ ref.residual_rows(Xr, phi, psi, a, e)
+            grad = grad + torch.autograd.grad(v, Xr)[0]
+        return dict(lam=lam, grad=grad)
+    d = _direction(m, X, rng)
+    dx = gpu(d["dx"])
+    jvp = torch.func.jvp(lambda Z: ref.residual_singular(Z, phi, psi), (Xg,), (dx,))[1].clone()
+    for a, e in ref.chunks():
+        jvp[a:e] += torch.func.jvp(lambda Z: ref.residual_rows(Z, phi, psi, a, e), (Xg,),
+                                   (dx,))[1]
+    jvp[ref.rows] = 0.0
+    _, rhs = ref.system(G, H, d["v"])
+    rhs = rhs[:, 0] - jvp
+    return dict(b=rhs, du=torch.linalg.solve(A, rhs))
