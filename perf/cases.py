@@ -116,8 +116,10 @@ def _mixed(box, block):
                           M.tri_block_mesh(n=block, centre=(3.0, 0.0, 0.0)))
 
 
-def _waves(X, rng, amplitude=2e-3):
-    """Points of z = 0 raised by a travelling wave of x and y (coincident dofs alike)."""
+def _waves(X, rng, nt):
+    """Points of z = 0 raised by a travelling wave of x and y (coincident dofs alike), by at
+    most 0.45 of the top layer's cell height (nt layers down to the draught 0.0625)."""
+    amplitude = min(2e-3, 0.3 * 0.0625 / nt)
     Y = X.copy()
     top = Y[:, 2] == 0.0
     p, q = rng.uniform(0.0, 2.0 * math.pi, 2)
@@ -135,7 +137,7 @@ def _setup(case, seed):
         return m, X, rng.standard_normal(m.n_dofs), 0.0, rng
     m = _flat_tank(*(case[k] for k in TANK))
     bc, speed = M.wigley_bc(m, seed=seed)
-    return m, _waves(m.support_points, rng), bc, speed, rng
+    return m, _waves(m.support_points, rng, case["nt"]), bc, speed, rng
 
 
 def _config(case):
