@@ -11,15 +11,18 @@
 // data is wave-uniform and arrives through scalar loads; each lane forms the 4+4 local G/H
 // values of the current cell for its row and adds them to register (G) and lane-private
 // LDS (H) accumulators, which leave through LDS as whole row segments, written once.
-//  * Strips (k_assemble_strips): on logically structured patches the wavefront sweeps a
-//    run of grid lines of at most 8 dofs; every cell is evaluated once per strip task it
-//    touches (about 1.1 times at 40k dofs) and its updates go to fixed slots.
+//  * Strips (k_assemble_strips): on logically structured patches a workgroup sweeps a run
+//    of grid lines of at most 8 dofs, four gaps between lines at a time; every cell is
+//    evaluated once per strip task it touches (about 1.1 times at 40k dofs) and its updates
+//    go to fixed slots.
 //  * Tiles (k_assemble_tiles): elsewhere, column tiles of up to TILE_COLS dofs and every
 //    cell touching the tile, with wave-uniform slot indices.
 // Both evaluate every cell with the regular rule; the singular kernel replaces the
 // regular part of each singular (row, cell) pair by its QGaussOneOverR integral.
 #include "wb_internal.h"
 #include "wb_device.h"
+
+#include <type_traits>
 
 namespace wb {
 
@@ -39,14 +42,29 @@ __device__ __forceinline__ double join_hilo(float hi, uint16_t lo)
     return (double)hi + (double)__uint_as_float((uint32_t)lo << 16);
 }
 
+// Factors from the sums of cell_local_values to the entries of G and H: 1/(4 pi), the sign
+// of H, and the powers of two of FAST's 2/r.
+template <bool FAST> struct RuleScale {
+    static constexpr double g = FAST ? 0.5 * INV4PI : INV4PI;
+    static constexpr double h = FAST ? -0.125 * INV4PI : -INV4PI;
+};
+
+// pointers to global memory that stay so through an opaque asm (a generic one would be stored
+// to with flat instructions)
+template <typename T> using glob = __attribute__((address_space(1))) T *;
+typedef glob<char> glob_bytes;
+
 // ------------------------------------------------------------------ cell geometry
 // deal.II FEValues<2,3> with a Q1 mapping: x = sum phi_k v_k, a = dx/dxi, b = dx/deta,
 // JxW = sqrt(det(J^T J)) w, n = orient (a x b)/|a x b|.
-// Record: y(3), n*JxW(3), JxW, xi*JxW (xi = first reference coordinate of the point).
+// Record: y(3), sn n*JxW(3), sj JxW, sj xi*JxW (xi = first reference coordinate of the
+// point).  sn = sj = 1, or the factors that make the strip kernel's sums the entries
+// themselves (RuleScale).
 __global__ void k_cell_geometry(const double *__restrict__ X, const int *__restrict__ cell_int,
                                 const int8_t *__restrict__ orient, int n_slots, int nq,
                                 const double *__restrict__ qpts, const double *__restrict__ qw,
-                                double *__restrict__ cellq, const int *__restrict__ slot_cell)
+                                double *__restrict__ cellq, const int *__restrict__ slot_cell,
+                                double sn, double sj)
 {
     const int gid = blockIdx.x * blockDim.x + threadIdx.x;
     if (gid >= n_slots * nq) return;
@@ -78,21 +96,24 @@ __global__ void k_cell_geometry(const double *__restrict__ X, const int *__restr
     r[0] = x[0];
     r[1] = x[1];
     r[2] = x[2];
-    r[3] = nn[0] * s * jxw;
-    r[4] = nn[1] * s * jxw;
-    r[5] = nn[2] * s * jxw;
-    r[6] = jxw;
-    r[7] = xi * jxw;
+    r[3] = nn[0] * s * jxw * sn;
+    r[4] = nn[1] * s * jxw * sn;
+    r[5] = nn[2] * s * jxw * sn;
+    r[6] = jxw * sj;
+    r[7] = xi * jxw * sj;
 }
 
 void launch_cell_geometry(const double *X, const int *cell_int, const int8_t *orient,
                           int n_slots, int nq, const double *qpts, const double *qw,
-                          double *cellq, hipStream_t s, const int *slot_cell)
+                          double *cellq, hipStream_t s, const int *slot_cell, int strip_precision)
 {
+    const bool fast = strip_precision == WB_PREC_FP32_IR;
+    const double sn = strip_precision < 0 ? 1.0 : fast ? RuleScale<true>::h : RuleScale<false>::h;
+    const double sj = strip_precision < 0 ? 1.0 : fast ? RuleScale<true>::g : RuleScale<false>::g;
     const long total = (long)n_slots * nq;
     if (total <= 0) return;
     hipLaunchKernelGGL(k_cell_geometry, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, X,
-                       cell_int, orient, n_slots, nq, qpts, qw, cellq, slot_cell);
+                       cell_int, orient, n_slots, nq, qpts, qw, cellq, slot_cell, sn, sj);
 }
 
 // ------------------------------------------------------------------ regular cells
@@ -110,60 +131,68 @@ void launch_cell_geometry(const double *X, const int *cell_int, const int8_t *or
 // registers 67 ms; 4 waves with the H tile in LDS 51 ms (the few spilled registers of the
 // 4-wave budget cost less than the lost occupancy).
 #ifndef WB_ASM_WAVES
-#define WB_ASM_WAVES 4  // requested waves per SIMD for the regular-cell kernel
+#define WB_ASM_WAVES 4  // requested waves per SIMD for the column-tile kernel
 #endif
-#ifndef WB_ASM_JUNROLL
-#define WB_ASM_JUNROLL 8  // unroll of the rule-row loop (>= Q: fully unrolled)
-#endif
-#ifndef WB_ASM_IUNROLL
-#define WB_ASM_IUNROLL 8  // unroll of the points of one rule row
-#endif
-#ifndef WB_ASM_BATCH
-#define WB_ASM_BATCH 4  // quadrature-point records per batch of scalar loads
-#endif
-#ifndef WB_ASM_HLDS
-#define WB_ASM_HLDS 1  // H accumulators in LDS (1) or in registers like G (0)
-#endif
-#define WB_STR(x) #x
-#define WB_UNROLL(n) _Pragma(WB_STR(unroll n))
 // The four local G and H values of one cell for the lane's collocation point x:
 // g_k = sum_q phi_k(q) JxW_q / |y_q - x|, h_k = sum_q phi_k(q) (y_q - x).N_q / |y_q - x|^3
-// (N = n JxW; the 1/(4 pi) factors and the sign of H are applied at the write-out).
+// (N = n JxW; the 1/(4 pi) factors and the sign of H are RuleScale's, applied at the tile
+// kernel's write-out and in the strip kernel's records).
 // rec: the cell's NQ records (wave-uniform, read by scalar loads).
 // FAST: the values are stored as FP32 hi + bf16 lo, and 1/r takes one Newton step
-// (rsqrt_f64_newton1) instead of the third-order one.
-template <int Q, bool FAST = false>
+// (rsqrt2_f64_newton1) instead of the third-order one; g then comes out times 2 and h
+// times 8 (RuleScale puts the powers of two back).
+// TOUCH: once a batch has arrived, one word of each 64-byte line of the next batch is touched (the
+// next cell's first records after the last batch; the arrays have REC_PAD records more),
+// so that the next batch finds its lines in the scalar cache: 27.5 -> 26.5 ms for the
+// FP32-IR assembly at 41k dofs.  A whole second batch does not fit the scalar registers.
+template <int Q, bool FAST, bool TOUCH>
 __device__ __forceinline__ void cell_local_values(const double *rec, double x0, double x1,
                                                   double x2, const PhiTable &nodes,
                                                   double (&g)[4], double (&h)[4])
 {
+    constexpr int B = Q <= 4 ? 4 : (Q + 1) / 2;  // points per batch of scalar loads
+    // larger rules keep their row loop: unrolled, they spill hundreds of registers
+    constexpr int JU = Q <= 4 ? Q : 1;
     double g0 = 0, g1 = 0, g2 = 0, g3 = 0, h0 = 0, h1 = 0, h2 = 0, h3 = 0;
-    WB_UNROLL(WB_ASM_JUNROLL)
+#pragma unroll JU
     for (int j = 0; j < Q; ++j) {
         double sg = 0, sg1 = 0, sh = 0, sh1 = 0;
-        // The records of WB_ASM_BATCH points arrive in one batch of scalar loads:
+        // The records of B points arrive in one batch of scalar loads:
         // scalar loads return out of order, so every use of one waits for all
         // outstanding ones (lgkmcnt(0)), and batching divides those waits.
-        WB_UNROLL(WB_ASM_IUNROLL)
-        for (int i = 0; i < Q; i += WB_ASM_BATCH) {
-            constexpr int B = WB_ASM_BATCH;
+#pragma unroll
+        for (int i = 0; i < Q; i += B) {
             double rr[8 * B];
 #pragma unroll
             for (int k = 0; k < 8 * B; ++k)
                 rr[k] = (i + k / 8 < Q) ? rec[(i + Q * j) * 8 + k] : 0.0;
+            int touch[B];
+            if constexpr (TOUCH) {
+                asm volatile("" ::"s"(rr[0]));  // the batch has arrived
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int k = 0; k < B; ++k)
+                    touch[k] = *(const int *)(rec + 8 * ((i + B < Q ? i + B : Q) + Q * j + k));
+                __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
             for (int u = 0; u < B; ++u) {
                 if (i + u >= Q) break;
                 const double *r = rr + 8 * u;
                 const double R0 = r[0] - x0, R1 = r[1] - x1, R2 = r[2] - x2;
                 const double r2 = __builtin_fma(R0, R0, __builtin_fma(R1, R1, R2 * R2));
-                const double ri = FAST ? rsqrt_f64_newton1(r2) : rsqrt_f64(r2);
+                const double ri = FAST ? rsqrt2_f64_newton1(r2) : rsqrt_f64(r2);
                 sg = __builtin_fma(ri, r[6], sg);   // sum JxW / r
                 sg1 = __builtin_fma(ri, r[7], sg1); // sum xi JxW / r
                 const double dn = __builtin_fma(R0, r[3], __builtin_fma(R1, r[4], R2 * r[5]));
                 const double thv = (dn * ri) * (ri * ri);
                 sh += thv;
                 sh1 = __builtin_fma(nodes.phi[i + u], thv, sh1);
+            }
+            if constexpr (TOUCH) {
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int k = 0; k < B; ++k) asm volatile("" ::"s"(touch[k]));
             }
         }
         const double sg0 = sg - sg1, sh0 = sh - sh1;  // sum (1 - xi_i) t
@@ -215,22 +244,14 @@ void k_assemble_tiles(
     const int t_end = min(n_tiles, t_begin + TILES_PER_WG);
     for (int tile = t_begin; tile < t_end; ++tile) {
         accv aG = 0.0;
-#if WB_ASM_HLDS
 #pragma unroll
         for (int c = 0; c < TC; ++c) lacc[c * ACC_LD + lane] = 0.0;
-#else
-        accv aH = 0.0;
-#endif
         // c is wave-uniform: the G vector index becomes an s_set_gpr_idx register move; the
         // H entry is a lane-private LDS word, updated by a no-return LDS add (ds_add_f64)
         auto upd = [&](int c, double g, double h) {
             aG[c & 15] += g;
-#if WB_ASM_HLDS
             __hip_atomic_fetch_add(&lacc[(c & 15) * ACC_LD + lane], h, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WAVEFRONT);
-#else
-            aH[c & 15] += h;
-#endif
         };
         double hs = 0.0;
         const int p0 = tile_ptr[tile], p1 = tile_ptr[tile + 1];
@@ -239,7 +260,7 @@ void k_assemble_tiles(
             const int cols = __builtin_amdgcn_readfirstlane(tile_cols[p]);
             const double *rec = cellq + (size_t)cell * (NQ * 8);
             double gl[4], hl[4];
-            cell_local_values<Q, OUT == 1>(rec, x0, x1, x2, nodes, gl, hl);
+            cell_local_values<Q, OUT == 1, false>(rec, x0, x1, x2, nodes, gl, hl);
             const double g0 = gl[0], g1 = gl[1], g2 = gl[2], g3 = gl[3];
             const double h0 = hl[0], h1 = hl[1], h2 = hl[2], h3 = hl[3];
             const int c0 = (int)(int8_t)(cols & 0xff);
@@ -269,17 +290,12 @@ void k_assemble_tiles(
         const int ncols = min(TC, tile_start[tile + 1] - c_begin);
 #pragma unroll
         for (int m = 1; m >= 0; --m) {
-            const double scale = m == 0 ? INV4PI : -INV4PI;
+            const double scale = m == 0 ? RuleScale<OUT == 1>::g : RuleScale<OUT == 1>::h;
             __syncthreads();
-#if WB_ASM_HLDS
             if (m == 0) {
 #pragma unroll
                 for (int c = 0; c < TC; ++c) lacc[c * ACC_LD + lane] = aG[c];
             }
-#else
-#pragma unroll
-            for (int c = 0; c < TC; ++c) lacc[c * ACC_LD + lane] = m == 0 ? aG[c] : aH[c];
-#endif
             __syncthreads();
             constexpr int RPI = TILE_ROWS / TC;  // rows per store instruction
             const int cl = lane % TC, rsub = lane / TC;
@@ -304,7 +320,7 @@ void k_assemble_tiles(
         }
         hs_total += hs;
     }
-    if (row < n) hsum_part[(size_t)tg * n + row] = hs_total * (-INV4PI);
+    if (row < n) hsum_part[(size_t)tg * n + row] = hs_total * RuleScale<OUT == 1>::h;
 }
 
 template <int Q>
@@ -352,60 +368,99 @@ void launch_assemble_tiles(int precision, int q_order, int tc, const double *xro
 }
 
 // ------------------------------------------------------------------ regular cells, strips
-// One wavefront owns 64 collocation rows (lane = row) and one strip task: the lines 0 ..
+// A workgroup owns 64 collocation rows (lane = row) and one strip task: the lines 0 ..
 // L - 1 (grid rows of at most STRIP_W consecutive dofs) of a run of levels of a structured
-// patch, swept gap by gap: gap t holds the cells between lines t and t + 1, t = -1 .. L - 1
-// (line -1 and line L belong to the neighbouring tasks).  Their records are built from
-// cell_int_s, whose vertex order puts the position direction first, so the cell at
-// position k of gap t adds its local values 0, 1 to positions k - 1, k of line t ("lo")
-// and 2, 3 to positions k - 1, k of line t + 1 ("up").  The position loop is unrolled, so
-// every update goes to a fixed register (G) or a fixed LDS offset (H, lane-private words).
-// After gap t, line t is complete: it is written once through LDS as whole row segments
-// and cleared, and the accumulators of line t + 1 become the "lo" ones of the next gap.
+// patch.  Gap t holds the cells between lines t and t + 1, t = -1 .. L - 1 (line -1 and line
+// L belong to the neighbouring tasks).  The records are built from cell_int_s, whose vertex
+// order puts the position direction first, so the cell at position k of gap t adds its local
+// values 0, 1 to positions k - 1, k of line t ("lo") and 2, 3 to positions k - 1, k of line
+// t + 1 ("up").
+//
+// The four wavefronts take four consecutive gaps at a time.  A wavefront walks its nine cell
+// positions (unrolled): G values add up in registers at fixed slots; an H value is complete
+// once the next position is done and goes straight to LDS.  Line t is then lo of gap t plus
+// up of gap t - 1 (the neighbouring wavefront's, or kept from the last round), and the four
+// lines leave together: 32 consecutive columns per row, so a store instruction fills whole
+// 128-byte lines (FP32: 2 rows x 32 columns).
+//
+// Bound: FP64 issue at the clock the power limit leaves (20.6 FP64 operations and one
+// v_rsq_f64 per point and row; at 41k dofs 93% of the issue slots at 2.08 GHz, where the one
+// wavefront per task form below had 76% at 2.06).  Measured at 41k dofs, FP32-IR / FP64:
+//   32.4 / 31.0 ms  one wavefront per task and 64 rows, one line (8 columns) stored at a time;
+//   28.8 / 28.4     with the next gap's records touched a gap ahead: the wavefronts of an XCD
+//                   walk a task side by side, and every new line made all of them wait for
+//                   one L2 miss;
+//   26.9 / 27.7     this form.  Without its stores it takes 22 ms: the 8-column segments left
+//                   the L2 2.3 times over (47.7 GB for 20.4 GB of entries; 34 GB now).
+// A small mesh gets four times as many wavefronts, each a quarter as long: 0.75 -> 0.19 ms
+// at 2,915 dofs, 0.27 -> 0.08 ms at 1,083.
+// Three wavefronts per SIMD hold everything in registers; at four, a spilled register reloaded
+// between the stores waits for all of them (loads and stores share one in-order counter).
+//
+// LDS, in regions of STRIP_W x 64 doubles: LO[4] by wavefront, UP[5] by gap modulo 5 (the
+// fifth is the last round's), and the G part's own kept UP: 10 x 4 KB, so that four
+// workgroups fill a CU's 160 KB.  Slot p of a region holds row r at (r ^ 2 p ^ 16 parity):
+// the write-out reads 16 columns (two lines of different parity) x 2 rows per half
+// wavefront from distinct banks.
 // Every cell is evaluated once per task it touches: once inside a strip, twice on the
 // boundary between two strips or two tasks of one strip.
-template <int K>
-__device__ __forceinline__ void strip_add(double (&lo)[STRIP_W], double (&up)[STRIP_W],
-                                          double *hlo, double *hup, const double (&g)[4],
-                                          const double (&h)[4], int acc_ld)
+constexpr int STRIP_REGION = STRIP_W * TILE_ROWS;  // doubles
+
+// The LDS word of position p for a row word of position 0 (byte offsets): slot p holds row
+// r at r ^ 2 p.  Opaque, so that the sixteen offsets of a gap are formed when needed and not
+// held in registers.
+__device__ __forceinline__ double *strip_word(double *lds, int word0, int p)
 {
-    if constexpr (K >= 1) {
-        lo[K - 1] += g[0];
-        up[K - 1] += g[2];
-        __hip_atomic_fetch_add(hlo + (K - 1) * acc_ld, h[0], __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_WAVEFRONT);
-        __hip_atomic_fetch_add(hup + (K - 1) * acc_ld, h[2], __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_WAVEFRONT);
-    }
-    if constexpr (K < STRIP_W) {
-        lo[K] += g[1];
-        up[K] += g[3];
-        __hip_atomic_fetch_add(hlo + K * acc_ld, h[1], __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_WAVEFRONT);
-        __hip_atomic_fetch_add(hup + K * acc_ld, h[3], __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_WAVEFRONT);
-    }
+    asm volatile("" : "+v"(word0));
+    return (double *)((char *)lds + ((word0 ^ (16 * p)) + 512 * p));
 }
 
-// The cells of one gap, positions K .. STRIP_W (present where cmask has the bit).
+// Positions K .. STRIP_W of one gap.  lo, up: G sums by position; wlo, wup: this lane's
+// words of position 0 of the H regions; cl, cu: H values of the previous cell still waiting
+// for this one; hs: the row sum of H over the positions of lines t (lm_lo) and t + 1 (lm_up)
+// that belong to the task.
 template <int Q, int K, bool FAST>
-__device__ __forceinline__ void strip_gap_cells(int cmask, const double *grec, double x0,
-                                                double x1, double x2, const PhiTable &nodes,
+__device__ __forceinline__ void strip_gap_cells(int cmask, int lm_lo, int lm_up,
+                                                const double *grec, double x0, double x1,
+                                                double x2, const PhiTable &nodes,
                                                 double (&lo)[STRIP_W], double (&up)[STRIP_W],
-                                                double *hlo, double *hup, int acc_ld)
+                                                double *lds, int wlo, int wup,
+                                                double cl, double cu, double &hs)
 {
     if constexpr (K <= STRIP_W) {
+        double nl = 0.0, nu = 0.0;
+        if constexpr (K < STRIP_W) lo[K] = up[K] = 0.0;
         if (cmask & (1 << K)) {
-            double cg[4], ch[4];
-            cell_local_values<Q, FAST>(grec + K * (Q * Q * 8), x0, x1, x2, nodes, cg, ch);
-            strip_add<K>(lo, up, hlo, hup, cg, ch, acc_ld);
+            double g[4], h[4];
+            cell_local_values<Q, FAST, true>(grec + K * (Q * Q * 8), x0, x1, x2, nodes, g, h);
+            if constexpr (K >= 1) {
+                lo[K - 1] += g[0];
+                up[K - 1] += g[2];
+                cl += h[0];
+                cu += h[2];
+            }
+            if constexpr (K < STRIP_W) {
+                lo[K] = g[1];
+                up[K] = g[3];
+            }
+            nl = h[1];
+            nu = h[3];
         }
-        strip_gap_cells<Q, K + 1, FAST>(cmask, grec, x0, x1, x2, nodes, lo, up, hlo, hup, acc_ld);
+        if constexpr (K >= 1) {
+            constexpr int P = K - 1;
+            *strip_word(lds, wlo, P) = cl;
+            *strip_word(lds, wup, P) = cu;
+            if (lm_lo & (1 << P)) hs += cl;
+            if (lm_up & (1 << P)) hs += cu;
+        }
+        strip_gap_cells<Q, K + 1, FAST>(cmask, lm_lo, lm_up, grec, x0, x1, x2, nodes, lo, up, lds,
+                                        wlo, wup, nl, nu, hs);
     }
 }
 
 template <int Q, int OUT>
-__global__ __launch_bounds__(TILE_ROWS) __attribute__((amdgpu_waves_per_eu(WB_ASM_WAVES)))
+__global__ __launch_bounds__(TILE_ROWS * STRIP_WAVES)
+__attribute__((amdgpu_waves_per_eu(3)))
 void k_assemble_strips(const double *__restrict__ xrow, const double *__restrict__ recs,
                        const int2 *__restrict__ tasks, const int4 *__restrict__ gaps, int n,
                        size_t ld, PhiTable nodes, void *__restrict__ Gv, void *__restrict__ Hv,
@@ -414,88 +469,167 @@ void k_assemble_strips(const double *__restrict__ xrow, const double *__restrict
 {
     constexpr int NQ = Q * Q;
     constexpr int KS = STRIP_W + 1;  // cell positions per gap
-    // H accumulators: two halves of STRIP_W lane-private columns [slot][lane], row stride
-    // ACC_LD; the half of line t + 1 follows the half of line t in turn
-    constexpr int ACC_LD = TILE_ROWS + 4;
-    __shared__ double lacc[2 * STRIP_W * ACC_LD];
-    const int lane = threadIdx.x;
-    const int rb = blockIdx.x;
+    constexpr int NW = STRIP_WAVES, NU = NW + 1;
+    static_assert(NW == 4 && STRIP_W == 8 && TILE_ROWS == 64, "the write-out's lane map");
+    __shared__ double lds[(NW + NU + 1) * STRIP_REGION];
+    // LO[wv], UP[gap % 5], UPG: G's UP of the last round's last gap
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row0 = blockIdx.x * TILE_ROWS;
     const int task = blockIdx.y;
-    const int row = rb * TILE_ROWS + lane;
+    const int row = row0 + lane;
     const int rr = row < n ? row : n - 1;
     const double x0 = xrow[3 * rr], x1 = xrow[3 * rr + 1], x2 = xrow[3 * rr + 2];
     const int2 T = tasks[task];
     const int g0 = __builtin_amdgcn_readfirstlane(T.x);
-    const int g1 = g0 + __builtin_amdgcn_readfirstlane(T.y);
-    double lo[STRIP_W], up[STRIP_W];
-#pragma unroll
-    for (int q = 0; q < STRIP_W; ++q) {
-        lo[q] = up[q] = 0.0;
-        lacc[q * ACC_LD + lane] = 0.0;
-        lacc[(STRIP_W + q) * ACC_LD + lane] = 0.0;
-    }
-    int hl = 0;  // LDS half of the lo line
+    const int ng = __builtin_amdgcn_readfirstlane(T.y);
+    // wait for the row's coordinates here: loads and stores share one in-order counter, so a
+    // wait for them inside the loop would wait for the last round's stores as well
+    asm volatile("" ::"v"(x0), "v"(x1), "v"(x2));
     double hs = 0.0;
-    // lane -> (position p, row offset rsub) in the write-out: each store instruction writes
-    // STRIP_W-column row segments of 64 / STRIP_W rows
-    constexpr int RPI = TILE_ROWS / STRIP_W;
-    const int wp = lane % STRIP_W, wsub = lane / STRIP_W;
-    for (int g = g0; g < g1; ++g) {
-        const int4 gi = gaps[g];
-        const int cmask = __builtin_amdgcn_readfirstlane(gi.x);
-        const int col0 = __builtin_amdgcn_readfirstlane(gi.y);
-        const int lmask = __builtin_amdgcn_readfirstlane(gi.z);
-        double *hlo = lacc + hl * (STRIP_W * ACC_LD) + lane;
-        double *hup = lacc + (1 - hl) * (STRIP_W * ACC_LD) + lane;
-        const double *grec = recs + (size_t)g * KS * (NQ * 8);
-        strip_gap_cells<Q, 0, OUT == 1>(cmask, grec, x0, x1, x2, nodes, lo, up, hlo, hup, ACC_LD);
-        // line t is complete: row sums, then H and G out through LDS, then clear
-        double *hbase = lacc + hl * (STRIP_W * ACC_LD);
+    auto line_mask = [&](int t) {  // positions of line t (the gap's index in the task)
+        return t < ng ? __builtin_amdgcn_readfirstlane(gaps[g0 + t].z) : 0;
+    };
+    int u5 = 0;  // (round's first gap) modulo 5
+    for (int j0 = 0; j0 < ng; j0 += NW) {
+        const int j = j0 + wv;  // this wavefront's gap
+        const int uw = (u5 + wv) % NU;
+        // this lane's words of position 0 in LO[wv] and UP[uw] (bytes)
+        const int wlo = 8 * (wv * STRIP_REGION + (lane ^ (16 * (wv & 1))));
+        const int wup = 8 * ((NW + uw) * STRIP_REGION + (lane ^ (16 * (uw & 1))));
+        double lo[STRIP_W], up[STRIP_W];
+        {
+            // touch the records of the wavefront's next gap (one word per 64-byte line): the
+            // wavefronts of an XCD walk the same task side by side, and without this each new
+            // line makes all of them wait for one L2 miss
+            constexpr int LINES = KS * NQ, PF = (LINES + 63) / 64;
+            float pf[PF];
+            const double *nrec = recs + (size_t)(g0 + min(j + NW, ng - 1)) * KS * (NQ * 8);
 #pragma unroll
-        for (int p = 0; p < STRIP_W; ++p)
-            if (lmask & (1 << p)) hs += hbase[p * ACC_LD + lane];
-        if (lmask) {
-            const bool present = (lmask >> wp) & 1;
-            const int col = col0 + __builtin_popcount(lmask & ((1 << wp) - 1));
+            for (int k = 0; k < PF; ++k)
+                pf[k] = *(const float *)(nrec + 8 * min(lane + 64 * k, LINES - 1));
+            int cmask = 0;
+            const double *grec = recs;
+            if (j < ng) {
+                cmask = __builtin_amdgcn_readfirstlane(gaps[g0 + j].x);
+                grec = recs + (size_t)(g0 + j) * KS * (NQ * 8);
+            }
+            strip_gap_cells<Q, 0, OUT == 1>(
+                cmask, line_mask(j), line_mask(j + 1), grec, x0, x1, x2, nodes, lo, up, lds, wlo,
+                wup, 0.0, 0.0, hs);
 #pragma unroll
-            for (int m = 1; m >= 0; --m) {  // H, then G
-                const double scale = m == 0 ? INV4PI : -INV4PI;
-                __syncthreads();
-                if (m == 0) {
+            for (int k = 0; k < PF; ++k) asm volatile("" ::"v"(pf[k]));
+        }
+        // Write-out: this lane's column c of the round's lines (line l, position pos) and
+        // row offset rsub; rows 16 wv .. 16 wv + 15, two per step.  The lane number is made
+        // opaque here so that none of this is held in registers across the cells: a register
+        // spilled there is reloaded between the stores, and each reload waits for them.
+        int ln = threadIdx.x & 63;
+        asm volatile("" : "+v"(ln));
+        const int c = (ln & 15) + 16 * (ln >> 5), rsub = (ln >> 4) & 1;
+        const int m0 = line_mask(j0), m1 = line_mask(j0 + 1), m2 = line_mask(j0 + 2),
+                  m3 = line_mask(j0 + 3);
+        int l = c >> 3, pos = c & 7, cols = 32;
+        if ((m0 & m1 & m2 & m3) != 255) {
+            const int e0 = __builtin_popcount(m0), e1 = e0 + __builtin_popcount(m1),
+                      e2 = e1 + __builtin_popcount(m2);
+            cols = e2 + __builtin_popcount(m3);
+            l = (c >= e0) + (c >= e1) + (c >= e2);
+            const int lm = l == 0 ? m0 : l == 1 ? m1 : l == 2 ? m2 : m3;
+            int rank = c - (l == 0 ? 0 : l == 1 ? e0 : l == 2 ? e1 : e2);
+            pos = 0;
 #pragma unroll
-                    for (int q = 0; q < STRIP_W; ++q) hbase[q * ACC_LD + lane] = lo[q];
-                    __syncthreads();
+            for (int p = 0; p < STRIP_W; ++p) {  // the position of the rank-th present dof
+                const int bit = (lm >> p) & 1;
+                if (bit && rank == 0) pos = p;
+                rank -= bit;
+            }
+        }
+        const int first = m0 ? 0 : m1 ? 1 : m2 ? 2 : 3;
+        const int col0 = j0 + first < ng ? __builtin_amdgcn_readfirstlane(gaps[g0 + j0 + first].y)
+                                         : 0;
+        int ul = u5 + l + NU - 1;  // UP region of gap j0 + l - 1
+        ul -= ul >= 2 * NU ? 2 * NU : ul >= NU ? NU : 0;
+        const int r0 = 16 * wv + rsub;  // this lane's first row in the block
+        // LDS bytes of (pos, r0); step it flips the row bits 2 it, which r0 leaves clear
+        const int plo = 8 * (l * STRIP_REGION + pos * TILE_ROWS + (r0 ^ (2 * pos) ^ (16 * (l & 1))));
+        const int pup = 8 * ((NW + ul) * STRIP_REGION + pos * TILE_ROWS +
+                             (r0 ^ (2 * pos) ^ (16 * (ul & 1))));
+        // line 0 finds G's up part of the last round in UPG
+        const int pug = l == 0 ? pup + 8 * (NU - ul) * STRIP_REGION : pup;
+        // the first gap of a task (line -1) has no line, so l = 0 of round 0 is never read
+        const int steps = c >= cols ? 0 : min(TILE_ROWS / (2 * NW), (n - row0 - r0 + 1) / 2);
+        // bytes of the lane's entry from the first row of the block (64 rows fit 32 bits) and
+        // wave-uniform row steps; the running row pointers are opaque, or their multiples
+        // of 2 ld would be kept (and spilled) over the cells
+        typedef typename std::conditional<OUT == 0, double, float>::type MT;
+        const unsigned vb = ((unsigned)r0 * (unsigned)ld + (unsigned)(col0 + c)) * sizeof(MT);
+        auto write_out = [&](int pu, void *Mb, uint16_t *Mlob) {
+            glob_bytes M = (glob_bytes)Mb + (size_t)row0 * ld * sizeof(MT);
+            glob_bytes Mlo = (glob_bytes)Mlob + (size_t)row0 * ld * 2;
+            // four steps' LDS reads in flight together
+            constexpr int NS = TILE_ROWS / (2 * NW), NB = 4;
+#pragma unroll
+            for (int ib = 0; ib < NS; ib += NB) {
+                double a[NB], b[NB];
+#pragma unroll
+                for (int k = 0; k < NB; ++k) {
+                    a[k] = *(const double *)((const char *)lds + (plo ^ (16 * (ib + k))));
+                    b[k] = *(const double *)((const char *)lds + (pu ^ (16 * (ib + k))));
                 }
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int r0 = 0; r0 < TILE_ROWS; r0 += RPI) {
-                    const int rl = r0 + wsub;
-                    const int grow = rb * TILE_ROWS + rl;
-                    if (grow < n && present) {
-                        const double v = hbase[wp * ACC_LD + rl] * scale;
-                        const size_t off = (size_t)grow * ld + col;
+                for (int k = 0; k < NB; ++k) {
+                    asm volatile("" : "+s"(M));
+                    if (OUT == 1) asm volatile("" : "+s"(Mlo));
+                    const double v = a[k] + b[k];
+                    if (ib + k < steps) {
                         if (OUT == 0) {
-                            ((double *)(m == 0 ? Gv : Hv))[off] = v;
+                            *(glob<MT>)(M + vb) = v;
                         } else {
                             float hi;
                             uint16_t lo16;
                             split_hilo(v, hi, lo16);
-                            ((float *)(m == 0 ? Gv : Hv))[off] = hi;
-                            (m == 0 ? Glo : Hlo)[off] = lo16;
+                            *(glob<MT>)(M + vb) = hi;
+                            *(glob<uint16_t>)(Mlo + vb / 2) = lo16;
                         }
                     }
+                    M += 2 * ld * sizeof(MT);
+                    Mlo += 4 * ld;
                 }
             }
-            __syncthreads();
-        }
+        };
+        __syncthreads();
+        write_out(pup, Hv, Hlo);
+        __syncthreads();
+        // G takes H's place; H's UP of the round's last gap stays for the next round, so G's
+        // goes to UPG once the last round's has been read
 #pragma unroll
-        for (int q = 0; q < STRIP_W; ++q) {
-            hbase[q * ACC_LD + lane] = 0.0;
-            lo[q] = up[q];
-            up[q] = 0.0;
+        for (int p = 0; p < STRIP_W; ++p) {
+            *strip_word(lds, wlo, p) = lo[p];
+            if (wv != NW - 1) *strip_word(lds, wup, p) = up[p];
         }
-        hl ^= 1;
+        __syncthreads();
+        write_out(pug, Gv, Glo);
+        __syncthreads();
+        if (wv == NW - 1) {
+            // with the parity of UP[uw], as line 0 of the next round reads it
+#pragma unroll
+            for (int p = 0; p < STRIP_W; ++p)
+                *strip_word(lds + (NU - uw) * STRIP_REGION, wup, p) = up[p];
+        }
+        u5 = (u5 + NW) % NU;
     }
-    if (row < n) hsum_part[(size_t)task * n + row] = hs * (-INV4PI);
+    // row sums of H, wavefront by wavefront
+    __syncthreads();
+    lds[threadIdx.x] = hs;
+    __syncthreads();
+    if (wv == 0 && row < n) {
+        double s = hs;
+#pragma unroll
+        for (int w = 1; w < NW; ++w) s += lds[w * 64 + lane];
+        hsum_part[(size_t)task * n + row] = s;
+    }
 }
 
 void launch_assemble_strips(int precision, int q_order, const double *xrow, const double *recs,
@@ -504,15 +638,15 @@ void launch_assemble_strips(int precision, int q_order, const double *xrow, cons
                             double *hsum_part, hipStream_t s)
 {
     if (n_tasks <= 0) return;
-    dim3 grid((n + TILE_ROWS - 1) / TILE_ROWS, n_tasks);
+    dim3 grid((n + TILE_ROWS - 1) / TILE_ROWS, n_tasks);  // row blocks of a task side by side
 #define WB_STRIPS(QV)                                                                          \
     case QV:                                                                                   \
         if (precision == WB_PREC_FP64)                                                         \
-            hipLaunchKernelGGL((k_assemble_strips<QV, 0>), grid, dim3(TILE_ROWS), 0, s, xrow,  \
+            hipLaunchKernelGGL((k_assemble_strips<QV, 0>), grid, dim3(TILE_ROWS * STRIP_WAVES), 0, s, xrow,  \
                                recs, (const int2 *)tasks, (const int4 *)gaps, n, ld, nodes, G, \
                                H, (uint16_t *)Glo, (uint16_t *)Hlo, hsum_part);                \
         else                                                                                   \
-            hipLaunchKernelGGL((k_assemble_strips<QV, 1>), grid, dim3(TILE_ROWS), 0, s, xrow,  \
+            hipLaunchKernelGGL((k_assemble_strips<QV, 1>), grid, dim3(TILE_ROWS * STRIP_WAVES), 0, s, xrow,  \
                                recs, (const int2 *)tasks, (const int4 *)gaps, n, ld, nodes, G, \
                                H, (uint16_t *)Glo, (uint16_t *)Hlo, hsum_part);                \
         break;

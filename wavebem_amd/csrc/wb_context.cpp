@@ -322,7 +322,7 @@ static void cell_records(wb_ctx *c)
         launch_cell_geometry(c->X.as<double>(), c->cell_int_s.as<int>(),
                              c->orient_s.as<int8_t>(), (int)c->plan.st_gcell.size(), nq,
                              c->qpts.as<double>(), c->qw.as<double>(), c->cellq_s.as<double>(),
-                             c->stream, c->st_gcell.as<int>());
+                             c->stream, c->st_gcell.as<int>(), c->cfg.precision);
         HIPCHK(hipGetLastError());
     }
 }
@@ -1883,8 +1883,8 @@ wb_status wb_set_mesh(wb_ctx *c, int n, int nc, const double *support, const int
             }
         upload(c->srule, rule.data(), rule.size(), s);
         const int nq = q.q_order * q.q_order;
-        c->cellq.ensure(sizeof(double) * 8 * (size_t)nq * nc);
-        c->cellq_s.ensure(sizeof(double) * 8 * (size_t)nq * (p.st_gcell.size() + 1));
+        c->cellq.ensure(sizeof(double) * 8 * ((size_t)nq * nc + REC_PAD));
+        c->cellq_s.ensure(sizeof(double) * 8 * ((size_t)nq * p.st_gcell.size() + REC_PAD));
         cell_records(c);
         alloc_matrices(c);
         c->hsum_part.ensure(sizeof(double) * (size_t)hsum_parts(c) * n);

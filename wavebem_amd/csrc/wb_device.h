@@ -15,18 +15,10 @@ namespace wb {
 #ifndef WB_RSQ_THIRD_ORDER
 #define WB_RSQ_THIRD_ORDER 1
 #endif
-#ifndef WB_RSQ_NEWTON1
-#define WB_RSQ_NEWTON1 0
-#endif
 __device__ __forceinline__ double rsqrt_f64(double r2)
 {
     double y = __builtin_amdgcn_rsq(r2);
-#if WB_RSQ_NEWTON1
-    // one Newton step: relative error (3/2) eps^2, about 4e-15 (4 operations)
-    const double h = 0.5 * r2;
-    const double e = __builtin_fma(-h, y * y, 0.5);
-    return __builtin_fma(y, e, y);
-#elif WB_RSQ_THIRD_ORDER
+#if WB_RSQ_THIRD_ORDER
     const double e = __builtin_fma(-r2, y * y, 1.0);
     const double p = __builtin_fma(0.375, e, 0.5);
     return __builtin_fma(y * e, p, y);
@@ -42,15 +34,15 @@ __device__ __forceinline__ double rsqrt_f64(double r2)
 #endif
 }
 
-// 1/sqrt(r2) with one Newton step from the hardware estimate: relative error (3/2) eps^2,
-// at most 4.1e-15 with the measured eps above (4 operations).  For values stored as FP32
-// hi + bf16 lo (relative rounding 2^-33 = 1.2e-10) this is 30000 times below the storage
-// error; the FP64 stores use rsqrt_f64.
-__device__ __forceinline__ double rsqrt_f64_newton1(double r2)
+// 2/sqrt(r2) with one Newton step y (3 - r2 y^2) from the hardware estimate: relative error
+// (3/2) eps^2, at most 4.1e-15 with the measured eps above (3 operations; the factor 2 goes
+// into the caller's scale, exactly).  For values stored as FP32 hi + bf16 lo (relative
+// rounding 2^-33 = 1.2e-10) this is 30000 times below the storage error; the FP64 stores
+// use rsqrt_f64.
+__device__ __forceinline__ double rsqrt2_f64_newton1(double r2)
 {
     const double y = __builtin_amdgcn_rsq(r2);
-    const double e = __builtin_fma(-0.5 * r2, y * y, 0.5);
-    return __builtin_fma(y, e, y);
+    return y * __builtin_fma(-r2, y * y, 3.0);
 }
 
 // Q1 shape values and reference derivatives at (xi, eta), deal.II vertex order

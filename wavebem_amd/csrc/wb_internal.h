@@ -47,10 +47,12 @@ void gauss_legendre_01(int n, double *x, double *w);
 // Strip schedule of the regular-cell assembly on logically structured patches.  A line
 // is at most STRIP_W dofs of one grid row, at consecutive positions; a strip is the lines
 // of one band of positions over consecutive grid rows ("levels"); a task is a run of
-// levels of one strip, swept by one wavefront per 64 collocation rows.  The cells of a
-// task lie between consecutive levels, so two lines at a time hold accumulators: the
-// ring of 2 STRIP_W slots, line l in half l & 1.
+// levels of one strip, swept by one workgroup per 64 collocation rows, its STRIP_WAVES
+// wavefronts taking that many consecutive gaps at a time.
 constexpr int STRIP_W = 8;
+constexpr int STRIP_WAVES = 4;
+// point records past the end of the record arrays that the assembly may touch (prefetch)
+constexpr int REC_PAD = 8;
 #ifndef WB_STRIP_TASK_ENTRIES
 #define WB_STRIP_TASK_ENTRIES 640
 #endif
@@ -193,7 +195,8 @@ std::string build_constraints(int n, const int *dn_ptr, const int *dn_idx, const
 // given (slots with -1 are left untouched).
 void launch_cell_geometry(const double *support_int, const int *cell_int, const int8_t *orient,
                           int n_slots, int nq, const double *qpts, const double *qw,
-                          double *cellq, hipStream_t s, const int *slot_cell = nullptr);
+                          double *cellq, hipStream_t s, const int *slot_cell = nullptr,
+                          int strip_precision = -1);  // wb_precision: records of the strip kernel
 void launch_assemble_tiles(int precision, int q_order, int tc, const double *xrow,
                            const double *cellq, const int *tile_ptr, const int *tile_cell,
                            const int *tile_cols, const int *tile_start, int n, int n_tiles,

@@ -323,7 +323,14 @@ bool build_strips(const std::vector<int> &cells, const std::vector<int> &dofs,
     const int ns = (Np + STRIP_W - 1) / STRIP_W;
     for (int s = 0; s < ns; ++s) {
         B.strip_first.push_back((int)B.order.size());
-        const int b0 = (int)((long)s * Np / ns), w = (int)((long)(s + 1) * Np / ns) - b0;
+        // whole strips of STRIP_W positions, so that full lines start at multiples of 8
+        // columns; a short rest (under half a strip) shares the last two strips evenly
+        const int rest = Np % STRIP_W, tail = rest && rest < STRIP_W / 2 && ns > 1;
+        const int b0 = tail && s == ns - 1 ? (s - 1) * STRIP_W + (STRIP_W + rest + 1) / 2
+                                           : s * STRIP_W;
+        const int b1 = s == ns - 1 ? Np
+                       : tail && s == ns - 2 ? b0 + (STRIP_W + rest + 1) / 2 : b0 + STRIP_W;
+        const int w = b1 - b0;
         auto cell_at = [&](int g, int k) {
             const int p0 = b0 + k - 1;
             if (p0 < 0 || p0 > Np - 2 || g < 0 || g > Na - 2) return -1;
@@ -333,11 +340,13 @@ bool build_strips(const std::vector<int> &cells, const std::vector<int> &dofs,
         for (int g = 0; g + 1 < Na; ++g)
             for (int k = 0; k <= w; ++k) total += cell_at(g, k) >= 0;
         int np = std::max(1, (int)std::lround((double)total / std::max(1, target)));
-        np = std::min(np, Na);
-        for (int r = 0; r < np; ++r) {
+        // L lines are L + 1 gaps: a multiple of the wavefronts that share them
+        int per = (Na + np - 1) / np;
+        per = (per + STRIP_WAVES) / STRIP_WAVES * STRIP_WAVES - 1;
+        for (int a0 = 0, a1; a0 < Na; a0 = a1) {
             // levels [a0, a1): gap t (task-local, -1 .. L-1) holds the cells between lines
             // t and t + 1; after it, line t is complete
-            const int a0 = (int)((long)r * Na / np), a1 = (int)((long)(r + 1) * Na / np);
+            a1 = std::min(Na, a0 + per);
             const int L = a1 - a0;
             const long cells_before = B.cells;
             B.tasks.push_back({(int)B.gaps.size(), L + 1, 0});
