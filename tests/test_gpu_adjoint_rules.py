@@ -1,0 +1,53 @@
+"""The tangent and the backward of the assembly over every rule order and ragged sizes: the
+two against each other, and directions that move only part of the mesh (pairs whose two
+sides stay are skipped) against the sum over the parts."""
+import numpy as np
+import pytest
+
+from wavebem_amd import mesh as M
+from wavebem_amd.bem import BEMProblem, Config
+
+pytestmark = pytest.mark.gpu
+
+
+def _state(n, q):
+    m = M.box_mesh(n=n, hi=(1.0, 0.8, 0.6), dirichlet_top=True)
+    p = BEMProblem(m, Config(quadrature_order=q))
+    p.assemble_system()
+    rng = np.random.default_rng(n * 10 + q)
+    phi, dphi, w = rng.standard_normal((3, m.n_dofs))
+    dx = rng.standard_normal((m.n_dofs, 3))
+    # coincident dofs move together, as a mesh does
+    _, first, inv = np.unique(np.round(m.support_points, 9), axis=0, return_index=True,
+                              return_inverse=True)
+    return m, p, phi, dphi, w, dx[first][np.asarray(inv).reshape(-1)]
+
+
+@pytest.mark.parametrize("q", [1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("n", [2, 7, 12])
+def test_tangent_and_backward_agree(n, q):
+    m, p, phi, dphi, w, dx = _state(n, q)
+    with p:
+        jv = p.residual_jvp(dx, phi, dphi, free_rows_only=False)
+        vj = p.residual_vjp(w, phi, dphi, free_rows_only=False)
+        top = m.support_points[:, 2] > 0.6 - 1e-9
+        some = np.where(top[:, None], dx, 0.0)
+        parts = (p.residual_jvp(some, phi, dphi, free_rows_only=False),
+                 p.residual_jvp(dx - some, phi, dphi, free_rows_only=False))
+        none = p.residual_jvp(np.zeros_like(dx), phi, dphi, free_rows_only=False)
+    # FP64 sums of up to 6 * 12^2 * 36 terms in two orders: 1e-13 each, with cancellation
+    a, b = w @ jv, (vj * dx).sum()
+    assert abs(a - b) < 1e-11 * np.abs(vj * dx).sum()
+    assert np.abs(parts[0] + parts[1] - jv).max() < 1e-11 * max(np.abs(x).max() for x in parts)
+    assert not none.any()
+
+
+def test_tangent_keeps_nan_of_parts_that_stay():
+    """0 * NaN: a NaN in phi reaches every row, also where neither row nor cell moves."""
+    m, p, phi, dphi, w, dx = _state(7, 4)
+    dx[m.support_points[:, 2] < 0.6 - 1e-9] = 0.0
+    bottom = np.flatnonzero((m.support_points[:, 2] < 1e-9))
+    phi[bottom[len(bottom) // 2]] = np.nan
+    with p:
+        jv = p.residual_jvp(dx, phi, dphi, free_rows_only=False)
+    assert np.isnan(jv).all()

@@ -29,13 +29,8 @@
 
 // Wave-uniform records (point records of a cell, row records) are read by scalar loads,
 // which return out of order: each use waits for every outstanding scalar load.  Records
-// are therefore fetched in batches, one wait per batch.
-#ifndef WB_ADJ_BATCH
-#define WB_ADJ_BATCH 4  // points (rows) per batch in k_vjp_rows and k_vjp_points
-#endif
-#ifndef WB_JVP_BATCH
-#define WB_JVP_BATCH 2  // points per batch in k_jvp_rows (18 doubles per point)
-#endif
+// are therefore fetched in batches, one wait per batch, and the next batch's lines touched
+// (one word each) while a batch is worked on; the arrays end in REC_PAD records of padding.
 
 namespace wb {
 
@@ -191,39 +186,112 @@ __global__ void k_constraint_T(int n_targets, const int *__restrict__ tgt,
     y[tgt[t]] = (T)s;
 }
 
-// Phi and Psi (Q1 interpolants of phi and psi) at every regular point of every cell
-__global__ void k_cell_state(int nc, int nq, const int *__restrict__ cell_int,
-                             const double *__restrict__ qpts, const double *__restrict__ phi,
-                             const double *__restrict__ psi, double *__restrict__ cstate)
+// Point records of the backward and the tangent: rec[c][q][8] = {y (3), N (3), Psi J, Phi}
+// (Phi, Psi the Q1 interpolants of phi and psi) and spsi[c][q] = Psi.  For a direction dX of
+// the vertices also trec[c][q][8] = {dy (3), dN (3), Psi dJ, N . dy},
+//   dy = sum sh_k dv_k, dc = da x b + a x db, dN = o w dc, dJ = w (c . dc) / |c|,
+// and moving[c]: 0 where the cell's vertices stay and its phi and psi are finite, so that
+// all of trec is zero (a pair of such a cell and a row that stays adds exactly nothing).
+__global__ void k_adj_records(int nc, int nq, const double *__restrict__ X,
+                              const double *__restrict__ dX, const int *__restrict__ cell_int,
+                              const int8_t *__restrict__ orient,
+                              const double *__restrict__ qpts, const double *__restrict__ qw,
+                              const double *__restrict__ cellq, const double *__restrict__ phi,
+                              const double *__restrict__ psi, double *__restrict__ rec,
+                              double *__restrict__ spsi, double *__restrict__ trec,
+                              int *__restrict__ moving)
 {
     const int gid = blockIdx.x * blockDim.x + threadIdx.x;
     if (gid >= nc * nq) return;
     const int c = gid / nq, q = gid % nq;
     double sh[4], dx[4], de[4];
     q1_shape(qpts[2 * q], qpts[2 * q + 1], sh, dx, de);
+    const double *cq = cellq + (size_t)gid * 8;
     double P = 0.0, S = 0.0;
+    bool finite = true;
     for (int k = 0; k < 4; ++k) {
         const int v = cell_int[4 * c + k];
         P += sh[k] * phi[v];
         S += sh[k] * psi[v];
+        finite = finite && isfinite(phi[v]) && isfinite(psi[v]);
     }
-    cstate[2 * (size_t)gid] = P;
-    cstate[2 * (size_t)gid + 1] = S;
+    double *r = rec + (size_t)gid * 8;
+    for (int d = 0; d < 6; ++d) r[d] = cq[d];
+    r[6] = S * cq[6];
+    r[7] = P;
+    spsi[gid] = S;
+    if (!dX) return;
+    double a[3] = {0, 0, 0}, b[3] = {0, 0, 0}, da[3] = {0, 0, 0}, db[3] = {0, 0, 0},
+           dy[3] = {0, 0, 0};
+    bool still = true;
+    for (int k = 0; k < 4; ++k) {
+        const int v = cell_int[4 * c + k];
+        for (int d = 0; d < 3; ++d) {
+            const double p = X[3 * v + d], dp = dX[3 * v + d];
+            still = still && dp == 0.0;
+            a[d] += dx[k] * p;
+            b[d] += de[k] * p;
+            da[d] += dx[k] * dp;
+            db[d] += de[k] * dp;
+            dy[d] += sh[k] * dp;
+        }
+    }
+    const double cx[3] = {a[1] * b[2] - a[2] * b[1], a[2] * b[0] - a[0] * b[2],
+                          a[0] * b[1] - a[1] * b[0]};
+    const double dc[3] = {da[1] * b[2] - da[2] * b[1] + a[1] * db[2] - a[2] * db[1],
+                          da[2] * b[0] - da[0] * b[2] + a[2] * db[0] - a[0] * db[2],
+                          da[0] * b[1] - da[1] * b[0] + a[0] * db[1] - a[1] * db[0]};
+    const double cl = sqrt(cx[0] * cx[0] + cx[1] * cx[1] + cx[2] * cx[2]);
+    const double so = orient[c] < 0 ? -1.0 : 1.0, w = qw[q];
+    double *t = trec + (size_t)gid * 8;
+    for (int d = 0; d < 3; ++d) {
+        t[d] = dy[d];
+        t[3 + d] = so * w * dc[d];
+    }
+    t[6] = S * (w * (cx[0] * dc[0] + cx[1] * dc[1] + cx[2] * dc[2]) / cl);
+    t[7] = cq[3] * dy[0] + cq[4] * dy[1] + cq[5] * dy[2];
+    if (q == 0) moving[c] = !(still && finite);
 }
+
+// One batch of B wave-uniform 8-double records: load, or touch (one word of each 64-byte line).
+template <int B> __device__ __forceinline__ void load_recs(const double *p, double (&r)[8 * B])
+{
+#pragma unroll
+    for (int k = 0; k < 8 * B; ++k) r[k] = p[k];
+}
+template <int B> __device__ __forceinline__ void touch_recs(const double *p, int (&t)[B])
+{
+#pragma unroll
+    for (int k = 0; k < B; ++k) t[k] = *(const int *)(p + 8 * k);
+}
+template <int B> __device__ __forceinline__ void touched(const int (&t)[B])
+{
+#pragma unroll
+    for (int k = 0; k < B; ++k) asm volatile("" ::"s"(t[k]));
+}
+
+// The four wavefronts of a workgroup (256 rows) walk the same cells, CG at a time in step,
+// so that they find each other's lines in the scalar cache, and touch the next group's
+// records in L2 (one word per 64-byte line) a group ahead: without that every new line makes
+// all wavefronts on the cells wait for one L2 miss.  A rule that does not fill its batches
+// keeps the loop over them (unrolled, it spills hundreds of scalar registers).
+constexpr int CG = 4;
 
 // Pass 1: part[chunk][row][3] = -w_i/(4 pi) sum over the chunk's regular (row, cell) pairs
 // of ds/dR (the x_i part of the backward).  Lane = row; cell data are wave-uniform.
+// Bound: FP64 issue, 28 operations and one v_rsq_f64 per pair and point; with
+// k_vjp_points 6.1 -> 4.9 ms at 11k dofs and 10.3k cells, 66 -> 59 at 41k (one wavefront per
+// workgroup, no touches).
 template <int Q>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_vjp_rows(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_vjp_rows(
     const double *__restrict__ xrow, const int *__restrict__ row_cls,
     const double *__restrict__ wrow, const double *__restrict__ phi,
-    const double *__restrict__ cellq, const double *__restrict__ cstate,
-    const int4 *__restrict__ cell_cls, int nc, int cells_per_chunk, int n,
-    double *__restrict__ part)
+    const double *__restrict__ recs, const int4 *__restrict__ cell_cls, int nc,
+    int cells_per_chunk, int n, double *__restrict__ part)
 {
-    constexpr int NQ = Q * Q;
-    const int lane = threadIdx.x;
-    const int row = blockIdx.x * 64 + lane;
+    constexpr int NQ = Q * Q, B = 4, BU = NQ % B == 0 ? NQ / B : 1;
+    const int lane = threadIdx.x & 63;
+    const int row = blockIdx.x * 256 + threadIdx.x;
     const int rr = row < n ? row : n - 1;
     const double x0 = xrow[3 * rr], x1 = xrow[3 * rr + 1], x2 = xrow[3 * rr + 2];
     const int rc = row_cls[rr];
@@ -231,44 +299,58 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     double acc0 = 0.0, acc1 = 0.0, acc2 = 0.0;
     const int c0 = blockIdx.y * cells_per_chunk;
     const int c1 = min(nc, c0 + cells_per_chunk);
-    if (__ballot(wi != 0.0) != 0) {
-        for (int c = c0; c < c1; ++c) {
-            const int4 cc = cell_cls[c];
-            const double *rec = cellq + (size_t)c * (NQ * 8);
-            const double *st = cstate + (size_t)c * (NQ * 2);
-            double g0 = 0.0, g1 = 0.0, g2 = 0.0;
-            constexpr int B = WB_ADJ_BATCH;
+    const bool live = __ballot(wi != 0.0) != 0;
+    for (int cb = c0; cb < c1; cb += CG) {
+        constexpr int PF = (CG * NQ + 63) / 64;
+        float pf[PF];
 #pragma unroll
-            for (int q0 = 0; q0 < NQ; q0 += B) {
-                double rb[8 * B], sb[2 * B];
+        for (int k = 0; k < PF; ++k)
+            pf[k] = *(const float *)(recs + 8 * (size_t)min((cb + CG) * NQ + lane + 64 * k,
+                                                            nc * NQ - 1));
+        if (live)
+            for (int c = cb; c < min(cb + CG, c1); ++c) {
+                const int4 cc = cell_cls[c];
+                const double *rec = recs + (size_t)c * (NQ * 8);
+                double g0 = 0.0, g1 = 0.0, g2 = 0.0;
+#pragma unroll BU
+                for (int q0 = 0; q0 < NQ; q0 += B) {
+                    double rb[8 * B];
+                    int tc[B];
+                    load_recs<B>(rec + 8 * q0, rb);
+                    asm volatile("" ::"s"(rb[0]));
+                    __builtin_amdgcn_sched_barrier(0);
+                    touch_recs<B>(rec + 8 * (q0 + B < NQ ? q0 + B : NQ), tc);
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int k = 0; k < 8 * B; ++k) rb[k] = (q0 + k / 8 < NQ) ? rec[8 * q0 + k] : 0.0;
-#pragma unroll
-                for (int k = 0; k < 2 * B; ++k) sb[k] = (q0 + k / 2 < NQ) ? st[2 * q0 + k] : 0.0;
-#pragma unroll
-                for (int u = 0; u < B; ++u) {
-                    if (q0 + u >= NQ) break;
-                    const double *r = rb + 8 * u;
-                    const double R0 = r[0] - x0, R1 = r[1] - x1, R2 = r[2] - x2;
-                    const double r2 = __builtin_fma(R0, R0, __builtin_fma(R1, R1, R2 * R2));
-                    const double ri = rsqrt_f64(r2);
-                    const double ri2 = ri * ri, ri3 = ri2 * ri, ri5 = ri3 * ri2;
-                    const double RN = __builtin_fma(R0, r[3], __builtin_fma(R1, r[4], R2 * r[5]));
-                    const double D = sb[2 * u] - phi_i;
-                    const double t1 = -D * ri3;
-                    const double t2 = __builtin_fma(3.0 * D * RN, ri5, sb[2 * u + 1] * r[6] * ri3);
-                    g0 = __builtin_fma(t1, r[3], __builtin_fma(t2, R0, g0));
-                    g1 = __builtin_fma(t1, r[4], __builtin_fma(t2, R1, g1));
-                    g2 = __builtin_fma(t1, r[5], __builtin_fma(t2, R2, g2));
+                    for (int u = 0; u < B; ++u) {
+                        if (q0 + u >= NQ) break;
+                        const double *r = rb + 8 * u;
+                        const double R0 = r[0] - x0, R1 = r[1] - x1, R2 = r[2] - x2;
+                        const double r2 = __builtin_fma(R0, R0, __builtin_fma(R1, R1, R2 * R2));
+                        const double ri = rsqrt_f64(r2);
+                        const double ri2 = ri * ri, ri3 = ri2 * ri;
+                        const double RN =
+                            __builtin_fma(R0, r[3], __builtin_fma(R1, r[4], R2 * r[5]));
+                        const double D = r[7] - phi_i;
+                        const double t1 = -(D * ri3);
+                        const double t2 = ri3 * __builtin_fma(3.0, D * (RN * ri2), r[6]);
+                        g0 = __builtin_fma(t1, r[3], __builtin_fma(t2, R0, g0));
+                        g1 = __builtin_fma(t1, r[4], __builtin_fma(t2, R1, g1));
+                        g2 = __builtin_fma(t1, r[5], __builtin_fma(t2, R2, g2));
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    touched<B>(tc);
+                }
+                const bool sing = (rc == cc.x) | (rc == cc.y) | (rc == cc.z) | (rc == cc.w);
+                if (!sing) {
+                    acc0 += g0;
+                    acc1 += g1;
+                    acc2 += g2;
                 }
             }
-            const bool sing = (rc == cc.x) | (rc == cc.y) | (rc == cc.z) | (rc == cc.w);
-            if (!sing) {
-                acc0 += g0;
-                acc1 += g1;
-                acc2 += g2;
-            }
-        }
+#pragma unroll
+        for (int k = 0; k < PF; ++k) asm volatile("" ::"v"(pf[k]));
+        __syncthreads();
     }
     if (row < n) {
         double *o = part + ((size_t)blockIdx.y * n + row) * 3;
@@ -281,68 +363,75 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
 
 // Pass 2: part[chunk][cell][q][7] = sum over the chunk's rows i (regular pairs only) of
 // w_i/(4 pi) (ds/dR (3), ds/dN (3), ds/dJ).  Lane = (cell, point); row data are
-// wave-uniform, packed as rowpack[i] = {x, y, z, w_i, phi_i, class}.
+// wave-uniform, packed as rowpack[i] = {x, y, z, w_i, phi_i, class, 0, 0}.  With the lane's N
+// and Psi constant, sum u1 N and sum -w Psi / r need one sum each.  Bound: FP64 issue, 31
+// operations and one v_rsq_f64 per pair and point.
 template <int Q>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_vjp_points(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_vjp_points(
     const double *__restrict__ rowpack, int n, int rows_per_chunk,
-    const double *__restrict__ cellq, const double *__restrict__ cstate,
+    const double *__restrict__ recs, const double *__restrict__ spsi,
     const int4 *__restrict__ cell_cls, int nc, double *__restrict__ part)
 {
     constexpr int NQ = Q * Q;
     constexpr int CPW = 64 / NQ;  // cells per wavefront
-    const int lane = threadIdx.x;
-    const int c = blockIdx.x * CPW + lane / NQ, q = lane % NQ;
+    constexpr int B = 4;          // rows per batch
+    const int lane = threadIdx.x & 63;
+    const int c = (blockIdx.x * 4 + (threadIdx.x >> 6)) * CPW + lane / NQ, q = lane % NQ;
     const bool live = lane < CPW * NQ && c < nc;
     const int cs = live ? c : 0;
-    const double *r = cellq + ((size_t)cs * NQ + q) * 8;
-    const double y0 = r[0], y1 = r[1], y2 = r[2], N0 = r[3], N1 = r[4], N2 = r[5], J = r[6];
-    const double P = cstate[2 * ((size_t)cs * NQ + q)], S = cstate[2 * ((size_t)cs * NQ + q) + 1];
+    const double *r = recs + ((size_t)cs * NQ + q) * 8;
+    const double y0 = r[0], y1 = r[1], y2 = r[2], N0 = r[3], N1 = r[4], N2 = r[5], SJ = r[6],
+                 P = r[7], S = spsi[(size_t)cs * NQ + q];
     const int4 cc = cell_cls[cs];
-    const double SJ = S * J;
-    double ay0 = 0, ay1 = 0, ay2 = 0, aN0 = 0, aN1 = 0, aN2 = 0, aJ = 0;
+    double ay0 = 0, ay1 = 0, ay2 = 0, aN0 = 0, aN1 = 0, aN2 = 0, s1 = 0, sr = 0;
     const int i0 = blockIdx.y * rows_per_chunk;
     const int i1 = min(n, i0 + rows_per_chunk);
-    constexpr int B = WB_ADJ_BATCH;
     for (int ib = i0; ib < i1; ib += B) {
         double pb[8 * B];
-#pragma unroll
-        for (int k = 0; k < 8 * B; ++k)
-            pb[k] = (ib + k / 8 < i1) ? rowpack[8 * (size_t)ib + k] : 0.0;
+        int tc[B];
+        load_recs<B>(rowpack + 8 * (size_t)ib, pb);
+        asm volatile("" ::"s"(pb[0]));
+        __builtin_amdgcn_sched_barrier(0);
+        touch_recs<B>(rowpack + 8 * ((size_t)ib + B), tc);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < B; ++u) {
             const double *rp = pb + 8 * u;
-            const double wi = rp[3];  // 0 for rows past the chunk (padding above)
-            if (wi == 0.0) continue;
+            const double wi = rp[3];
+            if (ib + u >= i1 || wi == 0.0) continue;  // past the chunk: another chunk's, or padding
             const int ci = (int)rp[5];
             const double R0 = y0 - rp[0], R1 = y1 - rp[1], R2 = y2 - rp[2];
             const double r2 = __builtin_fma(R0, R0, __builtin_fma(R1, R1, R2 * R2));
             const double ri = rsqrt_f64(r2);
-            const double ri2 = ri * ri, ri3 = ri2 * ri, ri5 = ri3 * ri2;
+            const double ri2 = ri * ri, ri3 = ri2 * ri;
             const double RN = __builtin_fma(R0, N0, __builtin_fma(R1, N1, R2 * N2));
             const double D = P - rp[4];
-            const double t1 = -D * ri3;
-            const double t2 = __builtin_fma(3.0 * D * RN, ri5, SJ * ri3);
             const bool sing = (ci == cc.x) | (ci == cc.y) | (ci == cc.z) | (ci == cc.w);
             const double ws = sing ? 0.0 : wi;
-            const double u1 = ws * t1, u2 = ws * t2;
-            ay0 = __builtin_fma(u1, N0, __builtin_fma(u2, R0, ay0));
-            ay1 = __builtin_fma(u1, N1, __builtin_fma(u2, R1, ay1));
-            ay2 = __builtin_fma(u1, N2, __builtin_fma(u2, R2, ay2));
+            const double wr3 = ws * ri3;
+            const double u1 = -(D * wr3);
+            const double u2 = wr3 * __builtin_fma(3.0, D * (RN * ri2), SJ);
+            s1 += u1;
+            ay0 = __builtin_fma(u2, R0, ay0);
+            ay1 = __builtin_fma(u2, R1, ay1);
+            ay2 = __builtin_fma(u2, R2, ay2);
             aN0 = __builtin_fma(u1, R0, aN0);
             aN1 = __builtin_fma(u1, R1, aN1);
             aN2 = __builtin_fma(u1, R2, aN2);
-            aJ = __builtin_fma(-ws * S, ri, aJ);
+            sr = __builtin_fma(ws, ri, sr);
         }
+        __builtin_amdgcn_sched_barrier(0);
+        touched<B>(tc);
     }
     if (live) {
         double *o = part + (((size_t)blockIdx.y * nc + c) * NQ + q) * 7;
-        o[0] = ay0 * INV4PI;
-        o[1] = ay1 * INV4PI;
-        o[2] = ay2 * INV4PI;
+        o[0] = __builtin_fma(s1, N0, ay0) * INV4PI;
+        o[1] = __builtin_fma(s1, N1, ay1) * INV4PI;
+        o[2] = __builtin_fma(s1, N2, ay2) * INV4PI;
         o[3] = aN0 * INV4PI;
         o[4] = aN1 * INV4PI;
         o[5] = aN2 * INV4PI;
-        o[6] = aJ * INV4PI;
+        o[6] = -S * sr * INV4PI;
     }
 }
 
@@ -473,109 +562,114 @@ __global__ __launch_bounds__(64) void k_vjp_singular(
 }
 
 // ------------------------------------------------------------------ tangent (JVP)
-// Directional derivatives of (y, N, J) at every regular point for vertex velocities dX:
-// dy = sum sh_k dv_k, dc = da x b + a x db, dN = o w dc, dJ = w (c . dc) / |c|.
-// trec[c][q][8] = {dy (3), dN (3), dJ, 0}.
-__global__ void k_tangent_points(int nc, int nq, const double *__restrict__ X,
-                                 const double *__restrict__ dX, const int *__restrict__ cell_int,
-                                 const int8_t *__restrict__ orient,
-                                 const double *__restrict__ qpts, const double *__restrict__ qw,
-                                 double *__restrict__ trec)
+// One cell's regular points in the tangent of the row with point x, velocity e and phi_i:
+//   sum_q ds/dR . d + ds/dN . dN + ds/dJ dJ   (without the 1/(4 pi)),   d = dy - e,
+// = sum_q 1/r^3 [ D (3 (R.N)(R.d)/r^2 - N.d - R.dN) + Psi J (R.d) ] - Psi dJ / r.
+// ROW: the row moves (e != 0); CELL: the cell does (its trec is not zero).
+template <int Q, bool ROW, bool CELL>
+__device__ __forceinline__ double jvp_cell(const double *rec, const double *tr, double x0,
+                                           double x1, double x2, double e0, double e1, double e2,
+                                           double phi_i)
 {
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= nc * nq) return;
-    const int c = gid / nq, q = gid % nq;
-    double sh[4], dx[4], de[4];
-    q1_shape(qpts[2 * q], qpts[2 * q + 1], sh, dx, de);
-    double a[3] = {0, 0, 0}, b[3] = {0, 0, 0}, da[3] = {0, 0, 0}, db[3] = {0, 0, 0},
-           dy[3] = {0, 0, 0};
-    for (int k = 0; k < 4; ++k) {
-        const int v = cell_int[4 * c + k];
-        for (int d = 0; d < 3; ++d) {
-            const double p = X[3 * v + d], dp = dX[3 * v + d];
-            a[d] += dx[k] * p;
-            b[d] += de[k] * p;
-            da[d] += dx[k] * dp;
-            db[d] += de[k] * dp;
-            dy[d] += sh[k] * dp;
+    constexpr int NQ = Q * Q, B = CELL ? 2 : 4, BU = NQ % B == 0 ? NQ / B : 1;
+    double g = 0.0;
+#pragma unroll BU
+    for (int q0 = 0; q0 < NQ; q0 += B) {
+        double rb[8 * B], tb[8 * B];
+        int tc[B], td[B];
+        load_recs<B>(rec + 8 * q0, rb);
+        if constexpr (CELL) load_recs<B>(tr + 8 * q0, tb);
+        asm volatile("" ::"s"(rb[0]));
+        __builtin_amdgcn_sched_barrier(0);
+        touch_recs<B>(rec + 8 * (q0 + B < NQ ? q0 + B : NQ), tc);
+        if constexpr (CELL) touch_recs<B>(tr + 8 * (q0 + B < NQ ? q0 + B : NQ), td);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+            if (q0 + u >= NQ) break;
+            const double *r = rb + 8 * u, *t = tb + 8 * u;
+            const double R0 = r[0] - x0, R1 = r[1] - x1, R2 = r[2] - x2;
+            const double r2 = __builtin_fma(R0, R0, __builtin_fma(R1, R1, R2 * R2));
+            const double ri = rsqrt_f64(r2);
+            const double ri2 = ri * ri, ri3 = ri2 * ri;
+            const double RN = __builtin_fma(R0, r[3], __builtin_fma(R1, r[4], R2 * r[5]));
+            const double D = r[7] - phi_i;
+            double Rd, a;  // R.d, N.d + R.dN
+            if constexpr (ROW) {
+                const double d0 = CELL ? t[0] - e0 : -e0, d1 = CELL ? t[1] - e1 : -e1,
+                             d2 = CELL ? t[2] - e2 : -e2;
+                Rd = __builtin_fma(R0, d0, __builtin_fma(R1, d1, R2 * d2));
+                a = __builtin_fma(r[3], d0, __builtin_fma(r[4], d1, r[5] * d2));
+            } else {
+                Rd = __builtin_fma(R0, t[0], __builtin_fma(R1, t[1], R2 * t[2]));
+                a = t[7];
+            }
+            if constexpr (CELL)
+                a = __builtin_fma(R0, t[3], __builtin_fma(R1, t[4], __builtin_fma(R2, t[5], a)));
+            const double v = __builtin_fma(3.0, (RN * ri2) * Rd, -a);
+            g = __builtin_fma(ri3, __builtin_fma(r[6], Rd, D * v), g);
+            if constexpr (CELL) g = __builtin_fma(-t[6], ri, g);
         }
+        __builtin_amdgcn_sched_barrier(0);
+        touched<B>(tc);
+        if constexpr (CELL) touched<B>(td);
     }
-    const double cx[3] = {a[1] * b[2] - a[2] * b[1], a[2] * b[0] - a[0] * b[2],
-                          a[0] * b[1] - a[1] * b[0]};
-    const double dc[3] = {da[1] * b[2] - da[2] * b[1] + a[1] * db[2] - a[2] * db[1],
-                          da[2] * b[0] - da[0] * b[2] + a[2] * db[0] - a[0] * db[2],
-                          da[0] * b[1] - da[1] * b[0] + a[0] * db[1] - a[1] * db[0]};
-    const double cl = sqrt(cx[0] * cx[0] + cx[1] * cx[1] + cx[2] * cx[2]);
-    const double so = orient[c] < 0 ? -1.0 : 1.0, w = qw[q];
-    double *t = trec + (size_t)gid * 8;
-    for (int d = 0; d < 3; ++d) {
-        t[d] = dy[d];
-        t[3 + d] = so * w * dc[d];
-    }
-    t[6] = w * (cx[0] * dc[0] + cx[1] * dc[1] + cx[2] * dc[2]) / cl;
-    t[7] = 0.0;
+    return g;
 }
 
-// part[chunk][row] = sum over the chunk's regular (row, cell) pairs of
-// ds/dR . (dy - dx_i) + ds/dN . dN + ds/dJ dJ  (without the 1/(4 pi)); lane = row.
+// part[chunk][row] = sum over the chunk's regular (row, cell) pairs of jvp_cell; lane = row.
+// A Newton direction moves the free surface only, so most pairs have a side that stays: a
+// wavefront whose rows all stay skips the cells that stay (their terms are exact zeros, for
+// finite phi and psi) and needs no d = dy - e for the others; a cell that stays costs the
+// moving rows half the record loads.  Bound: FP64 issue, 36 operations and one v_rsq_f64 per
+// pair and point where both sides move, 30 and 33 where one does.  At 41k dofs 36.3 -> 31.5 ms
+// with everything moving, 35.7 -> 21.2 with the free surface.
 template <int Q>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_jvp_rows(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_jvp_rows(
     const double *__restrict__ xrow, const double *__restrict__ dxrow,
     const int *__restrict__ row_cls, const double *__restrict__ phi,
-    const double *__restrict__ cellq, const double *__restrict__ cstate,
-    const double *__restrict__ trec, const int4 *__restrict__ cell_cls, int nc,
+    const double *__restrict__ recs, const double *__restrict__ trec,
+    const int *__restrict__ moving, const int4 *__restrict__ cell_cls, int nc,
     int cells_per_chunk, int n, double *__restrict__ part)
 {
     constexpr int NQ = Q * Q;
-    const int lane = threadIdx.x;
-    const int row = blockIdx.x * 64 + lane;
+    const int lane = threadIdx.x & 63;
+    const int row = blockIdx.x * 256 + threadIdx.x;
     const int rr = row < n ? row : n - 1;
     const double x0 = xrow[3 * rr], x1 = xrow[3 * rr + 1], x2 = xrow[3 * rr + 2];
     const double e0 = dxrow[3 * rr], e1 = dxrow[3 * rr + 1], e2 = dxrow[3 * rr + 2];
     const int rc = row_cls[rr];
     const double phi_i = phi[rr];
+    const bool row_moves =
+        __ballot(!(e0 == 0.0 && e1 == 0.0 && e2 == 0.0 && isfinite(phi_i))) != 0;
     double acc = 0.0;
     const int c0 = blockIdx.y * cells_per_chunk;
     const int c1 = min(nc, c0 + cells_per_chunk);
-    for (int c = c0; c < c1; ++c) {
-        const int4 cc = cell_cls[c];
-        const double *rec = cellq + (size_t)c * (NQ * 8);
-        const double *st = cstate + (size_t)c * (NQ * 2);
-        const double *tr = trec + (size_t)c * (NQ * 8);
-        double g = 0.0;
-        constexpr int B = WB_JVP_BATCH;
+    for (int cb = c0; cb < c1; cb += CG) {
+        constexpr int PF = (CG * NQ + 63) / 64;
+        float pf[2 * PF];
 #pragma unroll
-        for (int q0 = 0; q0 < NQ; q0 += B) {
-          double rb[8 * B], tb[8 * B], sb[2 * B];
-#pragma unroll
-          for (int k = 0; k < 8 * B; ++k) {
-              rb[k] = (q0 + k / 8 < NQ) ? rec[8 * q0 + k] : 0.0;
-              tb[k] = (q0 + k / 8 < NQ) ? tr[8 * q0 + k] : 0.0;
-          }
-#pragma unroll
-          for (int k = 0; k < 2 * B; ++k) sb[k] = (q0 + k / 2 < NQ) ? st[2 * q0 + k] : 0.0;
-#pragma unroll
-          for (int u = 0; u < B; ++u) {
-            if (q0 + u >= NQ) break;
-            const int q = u;  // index into this batch
-            const double *r = rb + 8 * u, *t = tb + 8 * u;
-            const double R0 = r[0] - x0, R1 = r[1] - x1, R2 = r[2] - x2;
-            const double r2 = __builtin_fma(R0, R0, __builtin_fma(R1, R1, R2 * R2));
-            const double ri = rsqrt_f64(r2);
-            const double ri2 = ri * ri, ri3 = ri2 * ri, ri5 = ri3 * ri2;
-            const double RN = __builtin_fma(R0, r[3], __builtin_fma(R1, r[4], R2 * r[5]));
-            const double D = sb[2 * q] - phi_i, E = sb[2 * q + 1];
-            const double t1 = -D * ri3;
-            const double t2 = __builtin_fma(3.0 * D * RN, ri5, E * r[6] * ri3);
-            const double d0 = t[0] - e0, d1 = t[1] - e1, d2 = t[2] - e2;  // dR
-            const double Nd = __builtin_fma(r[3], d0, __builtin_fma(r[4], d1, r[5] * d2));
-            const double Rd = __builtin_fma(R0, d0, __builtin_fma(R1, d1, R2 * d2));
-            const double RdN = __builtin_fma(R0, t[3], __builtin_fma(R1, t[4], R2 * t[5]));
-            g += t1 * (Nd + RdN) + t2 * Rd - E * ri * t[6];
-          }
+        for (int k = 0; k < PF; ++k) {
+            const size_t l = min((cb + CG) * NQ + lane + 64 * k, nc * NQ - 1);
+            pf[2 * k] = *(const float *)(recs + 8 * l);
+            pf[2 * k + 1] = *(const float *)(trec + 8 * l);
         }
-        const bool sing = (rc == cc.x) | (rc == cc.y) | (rc == cc.z) | (rc == cc.w);
-        if (!sing) acc += g;
+        for (int c = cb; c < min(cb + CG, c1); ++c) {
+            const int mv = moving[c];
+            if (!mv && !row_moves) continue;
+            const int4 cc = cell_cls[c];
+            const double *rec = recs + (size_t)c * (NQ * 8);
+            const double *tr = trec + (size_t)c * (NQ * 8);
+            const double g =
+                !mv ? jvp_cell<Q, true, false>(rec, tr, x0, x1, x2, e0, e1, e2, phi_i)
+                : row_moves ? jvp_cell<Q, true, true>(rec, tr, x0, x1, x2, e0, e1, e2, phi_i)
+                            : jvp_cell<Q, false, true>(rec, tr, x0, x1, x2, e0, e1, e2, phi_i);
+            const bool sing = (rc == cc.x) | (rc == cc.y) | (rc == cc.z) | (rc == cc.w);
+            if (!sing) acc += g;
+        }
+#pragma unroll
+        for (int k = 0; k < 2 * PF; ++k) asm volatile("" ::"v"(pf[k]));
+        __syncthreads();
     }
     if (row < n) part[(size_t)blockIdx.y * n + row] = acc;
 }
@@ -723,8 +817,24 @@ void launch_constraint_T(int is_float, int n_targets, const int *tgt, const int 
                            s, n_targets, tgt, ptr, src, coef, (const double *)x, (double *)y);
 }
 
-int vjp_row_chunks(int nc) { return max(1, min(64, (nc + 511) / 512)); }
-int vjp_point_chunks(int n) { return max(1, min(16, (n + 4095) / 4096)); }
+// Chunks of the cells for the row passes: at least 2048 workgroups of 256 rows (a CU holds
+// four), at most 1024 cells and at least 16 in a chunk.
+int vjp_row_chunks(int n, int nc)
+{
+    const int blocks = (n + 255) / 256;
+    const int want = max((nc + 1023) / 1024, (2048 + blocks - 1) / blocks);
+    return max(1, min(want, (nc + 15) / 16));
+}
+// Chunks of the rows for the point pass, likewise: at least 2048 workgroups of four
+// wavefronts, at least 128 rows in a chunk.
+int vjp_point_chunks(int n, int nc, int nq)
+{
+    const int blocks = (nc + 4 * (64 / nq) - 1) / (4 * (64 / nq));
+    const int want = max((n + 4095) / 4096, (2048 + blocks - 1) / blocks);
+    return max(1, min(want, (n + 127) / 128));
+}
+// doubles of the point records (with padding) and of Psi after them
+size_t adj_record_doubles(int nc, int nq) { return 8 * ((size_t)nc * nq + REC_PAD); }
 
 void launch_residual_vjp(int q_order, int n, int nc, const double *X, const int *row_cls,
                          const double *wrow, const double *phi, const double *psi,
@@ -736,19 +846,21 @@ void launch_residual_vjp(int q_order, int n, int nc, const double *X, const int 
                          double *xs, double *spart, hipStream_t s)
 {
     const int nq = q_order * q_order;
-    hipLaunchKernelGGL(k_cell_state, dim3((nc * nq + 255) / 256), dim3(256), 0, s, nc, nq,
-                       cell_int, qpts, phi, psi, cstate);
-    const int rch = vjp_row_chunks(nc), cpc = (nc + rch - 1) / rch;
-    const int pch = vjp_point_chunks(n), rpc = (n + pch - 1) / pch;
-    dim3 g1((n + 63) / 64, rch);
-    const int cpw = 64 / nq;
+    double *spsi = cstate + adj_record_doubles(nc, nq);
+    hipLaunchKernelGGL(k_adj_records, dim3((nc * nq + 255) / 256), dim3(256), 0, s, nc, nq, X,
+                       (const double *)nullptr, cell_int, orient, qpts, qw, cellq, phi, psi,
+                       cstate, spsi, (double *)nullptr, (int *)nullptr);
+    const int rch = vjp_row_chunks(n, nc), cpc = (nc + rch - 1) / rch;
+    const int pch = vjp_point_chunks(n, nc, nq), rpc = (n + pch - 1) / pch;
+    dim3 g1((n + 255) / 256, rch);
+    const int cpw = 4 * (64 / nq);
     dim3 g2((nc + cpw - 1) / cpw, pch);
 #define WB_VJP(QV)                                                                          \
     case QV:                                                                                \
-        hipLaunchKernelGGL(k_vjp_rows<QV>, g1, dim3(64), 0, s, X, row_cls, wrow, phi, cellq,  \
-                           cstate, (const int4 *)cell_cls, nc, cpc, n, part1);               \
-        hipLaunchKernelGGL(k_vjp_points<QV>, g2, dim3(64), 0, s, rowpack, n, rpc, cellq,      \
-                           cstate, (const int4 *)cell_cls, nc, part2);                       \
+        hipLaunchKernelGGL(k_vjp_rows<QV>, g1, dim3(256), 0, s, X, row_cls, wrow, phi, cstate, \
+                           (const int4 *)cell_cls, nc, cpc, n, part1);                       \
+        hipLaunchKernelGGL(k_vjp_points<QV>, g2, dim3(256), 0, s, rowpack, n, rpc, cstate,    \
+                           spsi, (const int4 *)cell_cls, nc, part2);                         \
         break;
     switch (q_order) {
         WB_VJP(1)
@@ -777,16 +889,16 @@ void launch_residual_jvp(int q_order, int n, int nc, const double *X, const doub
                          double *trec, double *part, double *ds, double *out, hipStream_t s)
 {
     const int nq = q_order * q_order;
-    hipLaunchKernelGGL(k_cell_state, dim3((nc * nq + 255) / 256), dim3(256), 0, s, nc, nq,
-                       cell_int, qpts, phi, psi, cstate);
-    hipLaunchKernelGGL(k_tangent_points, dim3((nc * nq + 255) / 256), dim3(256), 0, s, nc, nq,
-                       X, dX, cell_int, orient, qpts, qw, trec);
-    const int rch = vjp_row_chunks(nc), cpc = (nc + rch - 1) / rch;
-    dim3 g1((n + 63) / 64, rch);
+    double *spsi = cstate + adj_record_doubles(nc, nq);
+    int *moving = (int *)(trec + adj_record_doubles(nc, nq));
+    hipLaunchKernelGGL(k_adj_records, dim3((nc * nq + 255) / 256), dim3(256), 0, s, nc, nq, X, dX,
+                       cell_int, orient, qpts, qw, cellq, phi, psi, cstate, spsi, trec, moving);
+    const int rch = vjp_row_chunks(n, nc), cpc = (nc + rch - 1) / rch;
+    dim3 g1((n + 255) / 256, rch);
 #define WB_JVP(QV)                                                                          \
     case QV:                                                                                \
-        hipLaunchKernelGGL(k_jvp_rows<QV>, g1, dim3(64), 0, s, X, dX, row_cls, phi, cellq,    \
-                           cstate, trec, (const int4 *)cell_cls, nc, cpc, n, part);          \
+        hipLaunchKernelGGL(k_jvp_rows<QV>, g1, dim3(256), 0, s, X, dX, row_cls, phi, cstate,  \
+                           trec, moving, (const int4 *)cell_cls, nc, cpc, n, part);          \
         break;
     switch (q_order) {
         WB_JVP(1)

@@ -2637,7 +2637,7 @@ wb_status wb_residual_vjp(wb_ctx *c, const double *w, const double *phi, const d
         HIPCHK(hipMemcpyAsync(xs_host.data(), c->X.p, sizeof(double) * 3 * n,
                               hipMemcpyDeviceToHost, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
-        std::vector<double> rp(8 * (size_t)n, 0.0);
+        std::vector<double> rp(8 * ((size_t)n + REC_PAD), 0.0);
         for (int i = 0; i < n; ++i) {
             for (int d = 0; d < 3; ++d) rp[8 * i + d] = xs_host[3 * i + d];
             rp[8 * i + 3] = wi[i];
@@ -2649,9 +2649,10 @@ wb_status wb_residual_vjp(wb_ctx *c, const double *w, const double *phi, const d
         upload(c->vjp_psi, si.data(), n, c->stream);
         upload(c->vjp_rows, rp.data(), rp.size(), c->stream);
         const int npairs = (int)c->plan.sing_cell.size();
-        c->vjp_cstate.ensure(sizeof(double) * 2 * (size_t)nc * nq);
-        c->vjp_p1.ensure(sizeof(double) * 3 * (size_t)vjp_row_chunks(nc) * n);
-        c->vjp_p2.ensure(sizeof(double) * 7 * (size_t)vjp_point_chunks(n) * nc * nq);
+        // point records and Psi
+        c->vjp_cstate.ensure(sizeof(double) * (adj_record_doubles(nc, nq) + (size_t)nc * nq));
+        c->vjp_p1.ensure(sizeof(double) * 3 * (size_t)vjp_row_chunks(n, nc) * n);
+        c->vjp_p2.ensure(sizeof(double) * 7 * (size_t)vjp_point_chunks(n, nc, nq) * nc * nq);
         c->vjp_xg.ensure(sizeof(double) * 3 * (size_t)n);
         c->vjp_vbar.ensure(sizeof(double) * 12 * (size_t)nc);
         c->vjp_xs.ensure(sizeof(double) * 3 * (size_t)n);
@@ -2720,9 +2721,10 @@ wb_status wb_residual_jvp(wb_ctx *c, const double *dx, const double *phi, const 
         upload(c->vjp_phi, pi.data(), n, c->stream);
         upload(c->vjp_psi, si.data(), n, c->stream);
         upload(c->vjp_w, dxi.data(), dxi.size(), c->stream);  // the direction, 3 per point
-        c->vjp_cstate.ensure(sizeof(double) * 2 * (size_t)nc * nq);
-        c->vjp_p2.ensure(sizeof(double) * 8 * (size_t)nc * nq);              // tangent records
-        c->vjp_p1.ensure(sizeof(double) * (size_t)vjp_row_chunks(nc) * n);   // row partials
+        // point records and Psi; tangent records and the cells' moving flags; row partials
+        c->vjp_cstate.ensure(sizeof(double) * (adj_record_doubles(nc, nq) + (size_t)nc * nq));
+        c->vjp_p2.ensure(sizeof(double) * adj_record_doubles(nc, nq) + sizeof(int) * (size_t)nc);
+        c->vjp_p1.ensure(sizeof(double) * (size_t)vjp_row_chunks(n, nc) * n);
         c->vjp_xs.ensure(sizeof(double) * n);                                // singular part
         c->vjp_xg.ensure(sizeof(double) * n);                                // result
         launch_residual_jvp(c->quad.q_order, n, nc, c->X.as<double>(), c->vjp_w.as<double>(),

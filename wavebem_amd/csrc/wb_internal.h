@@ -340,10 +340,12 @@ void launch_gemvT(int mode, const void *G, const void *H, const void *Glo, const
 void launch_constraint_T(int is_float, int n_targets, const int *tgt, const int *ptr,
                          const int *src, const double *coef, const void *x, void *y,
                          hipStream_t s);
-// backward of the assembly; buffer sizes: cstate nc*nq*2, part1 vjp_row_chunks(nc)*n*3,
-// part2 vjp_point_chunks(n)*nc*nq*7, xgrad n*3, vbar nc*12, xs n*3, spart n_sing*12
-int vjp_row_chunks(int nc);
-int vjp_point_chunks(int n);
+// backward of the assembly; buffer sizes: cstate adj_record_doubles + nc*nq,
+// part1 vjp_row_chunks*n*3,
+// part2 vjp_point_chunks*nc*nq*7, rowpack 8*(n + REC_PAD), xgrad n*3, vbar nc*12, xs n*3, spart n_sing*12
+int vjp_row_chunks(int n, int nc);
+int vjp_point_chunks(int n, int nc, int nq);
+size_t adj_record_doubles(int nc, int nq);
 void launch_residual_vjp(int q_order, int n, int nc, const double *X, const int *row_cls,
                          const double *wrow, const double *phi, const double *psi,
                          const double *rowpack, const double *cellq, const int *cell_int,
@@ -390,7 +392,8 @@ void launch_permute(int n, const int *idx, const double *src, double *dst, int g
                     hipStream_t s);
 
 // tangent of the residual: out[i] = sum_d dR_i/dx_d . dX_d (0 on rows flagged in skip);
-// buffers: cstate nc*nq*2, trec nc*nq*8, part vjp_row_chunks(nc)*n, ds n, out n
+// buffers: cstate adj_record_doubles + nc*nq, trec adj_record_doubles and nc ints, part
+// vjp_row_chunks*n, ds n, out n
 void launch_residual_jvp(int q_order, int n, int nc, const double *X, const double *dX,
                          const int *row_cls, const double *phi, const double *psi,
                          const double *cellq, const int *cell_int, const int *cell_cls,
