@@ -123,7 +123,7 @@ struct wb_ctx {
     DevBuf vjp_w, vjp_phi, vjp_psi, vjp_rows, vjp_cstate, vjp_p1, vjp_p2, vjp_xg, vjp_vbar,
         vjp_xs, vjp_spart;
     // L2 projections: node -> (cell, local vertex) incidence, element blocks, CG vectors
-    DevBuf inc_ptr, inc_item, pj_emass, pj_erhs, pj_u, pj_psi, pj_B, pj_X, pj_R, pj_Z, pj_P,
+    DevBuf inc_ptr, inc_item, pj_emass, pj_erhs, pj_u, pj_psi, pj_B, pj_X, pj_R, pj_Z, pj_P, pj_Pb,
         pj_Q, pj_dinv, pj_part, pj_part2, pj_state;
     int proj_iterations = 0;
     int n_lines = 0, n_free = 0;
@@ -200,7 +200,7 @@ struct wb_ctx {
             &ct_ptr, &ct_src, &ct_coef, &gt_part, &vjp_w, &vjp_phi, &vjp_psi, &vjp_rows,
             &vjp_cstate, &vjp_p1, &vjp_p2, &vjp_xg, &vjp_vbar, &vjp_xs, &vjp_spart, &inc_ptr,
             &inc_item, &pj_emass, &pj_erhs, &pj_u, &pj_psi, &pj_B, &pj_X, &pj_R, &pj_Z, &pj_P,
-            &pj_Q, &pj_dinv, &pj_part, &pj_part2, &pj_state, &A16, &rs16, &hm_idx, &hm_size, &hm_seg,
+            &pj_Pb, &pj_Q, &pj_dinv, &pj_part, &pj_part2, &pj_state, &A16, &rs16, &hm_idx, &hm_size, &hm_seg,
             &hm_near, &hm_rank, &hm_scale, &hm_Y, &hm_Mx, &hm_Q, &hm_B, &hm_D, &hm_doff, &hm_T,
             &hm_part, &hm_iptr, &hm_items, &hm_pos};
         for (DevBuf *b : mw.all()) v.push_back(b);
@@ -1152,7 +1152,9 @@ static void project_fields(wb_ctx *c, const double *u, int normalize, double *no
     const size_t v6 = sizeof(double) * 6 * (size_t)n;
     c->pj_emass.ensure(sizeof(double) * 10 * (size_t)nc);
     c->pj_erhs.ensure(sizeof(double) * 24 * (size_t)nc);
-    for (DevBuf *b : {&c->pj_B, &c->pj_X, &c->pj_R, &c->pj_Z, &c->pj_P, &c->pj_Q}) b->ensure(v6);
+    for (DevBuf *b :
+         {&c->pj_B, &c->pj_X, &c->pj_R, &c->pj_Z, &c->pj_P, &c->pj_Pb, &c->pj_Q})
+        b->ensure(v6);
     c->pj_dinv.ensure(sizeof(double) * n);
     const int nb = proj_blocks(n);
     c->pj_part.ensure(sizeof(double) * 6 * nb);
@@ -1173,12 +1175,13 @@ static void project_fields(wb_ctx *c, const double *u, int normalize, double *no
         pd = c->pj_psi.as<double>();
     }
     double *X = c->pj_X.as<double>(), *R = c->pj_R.as<double>(), *Z = c->pj_Z.as<double>(),
-           *P = c->pj_P.as<double>(), *Q = c->pj_Q.as<double>(), *st = c->pj_state.as<double>();
+           *Q = c->pj_Q.as<double>(), *st = c->pj_state.as<double>();
+    double *const P[2] = {c->pj_P.as<double>(), c->pj_Pb.as<double>()};
     launch_proj_setup(c->X.as<double>(), c->cell_int.as<int>(), c->orient.as<int8_t>(), ud, pd,
                       nc, nq, c->qpts.as<double>(), c->qw.as<double>(), c->inc_ptr.as<int>(),
                       c->inc_item.as<int>(), n, c->pj_emass.as<double>(),
                       c->pj_erhs.as<double>(), c->pj_B.as<double>(), c->pj_dinv.as<double>(), s);
-    launch_proj_cg_start(c->pj_B.as<double>(), c->pj_dinv.as<double>(), n, X, R, Z, P,
+    launch_proj_cg_start(c->pj_B.as<double>(), c->pj_dinv.as<double>(), n, X, R, Z,
                          c->pj_part2.as<double>(), st, s);
     HIPCHK(hipGetLastError());
     const double tol = 1e-14;
@@ -1197,6 +1200,7 @@ static void project_fields(wb_ctx *c, const double *u, int normalize, double *no
                                 c->cell_int.as<int>(), c->pj_emass.as<double>(),
                                 c->pj_dinv.as<double>(), n, it, X, R, Z, P, Q,
                                 c->pj_part.as<double>(), c->pj_part2.as<double>(), st, s);
+        launch_proj_cg_state(c->pj_part2.as<double>(), n, it, st, s);
         HIPCHK(hipGetLastError());
     }
     c->proj_iterations = it;

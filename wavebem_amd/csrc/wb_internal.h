@@ -226,11 +226,12 @@ void launch_proj_setup(const double *X, const int *cell_int, const int8_t *orien
                        const double *qw, const int *inc_ptr, const int *inc_item, int n,
                        double *emass, double *erhs, double *B, double *dinv, hipStream_t s);
 void launch_proj_cg_start(const double *B, const double *dinv, int n, double *Xs, double *R,
-                          double *Z, double *P, double *part2, double *state, hipStream_t s);
+                          double *Z, double *part2, double *state, hipStream_t s);
 void launch_proj_cg_iter(const int *inc_ptr, const int *inc_item, const int *cell_int,
                          const double *emass, const double *dinv, int n, int iter, double *Xs,
-                         double *R, double *Z, double *P, double *Q, double *part,
+                         double *R, double *Z, double *const P[2], double *Q, double *part,
                          double *part2, double *state, hipStream_t s);
+void launch_proj_cg_state(const double *part2, int n, int iter, double *state, hipStream_t s);
 void launch_alpha_reduce(const double *hsum_part, int n_parts, const double *hsum_sing, int n,
                          double *alpha, hipStream_t s);
 
