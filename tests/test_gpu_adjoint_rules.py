@@ -7,7 +7,7 @@ import pytest
 from wavebem_amd import mesh as M
 from wavebem_amd.bem import BEMProblem, Config
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("gpu_available")]
 
 
 def _state(n, q):

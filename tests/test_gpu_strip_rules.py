@@ -9,7 +9,7 @@ from tests import helpers as T
 from wavebem_amd import mesh as M
 from wavebem_amd.bem import BEMProblem, Config
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("gpu_available")]
 
 
 @pytest.mark.parametrize("precision,bar", [("fp64", 1e-10), ("fp32_ir", 1e-9)])
