@@ -395,16 +395,21 @@ static void ensure_work(wb_ctx *c)
     }
 }
 
+// with the compressed inner operator, a new basis vector also goes to the product's
+// cluster-order copy, so its product needs no gather
+static bool cluster_copy(const wb_ctx *c, int is_float)
+{
+    return is_float && c->float_mode == 4 &&
+           c->hm_T.bytes >= sizeof(float) * (size_t)c->hmp.ncl * HM_CL;
+}
+
 // Launch of k_finalize that also publishes the column as publication seq
 static void finalize_publish(wb_ctx *c, int is_float, int kcount, const double *h1,
                              const double *h2, void *z, int n, void *vout,
                              unsigned long long seq)
 {
     double *slot = c->hmap_dev + (seq & 1) * HMAP_STRIDE;
-    // with the compressed inner operator, the new basis vector also goes to the product's
-    // cluster-order copy, so its product needs no gather
-    const bool xc = is_float && c->float_mode == 4 && c->hm_T.bytes >= sizeof(float) *
-                                                                         (size_t)c->hmp.ncl * HM_CL;
+    const bool xc = cluster_copy(c, is_float);
     launch_finalize(is_float, kcount, h1, h2, c->Pn.as<double>(), z, n, vout,
                     c->hbuf.as<double>(), c->stream, 1, 0, 0, 0, 0, nullptr, slot,
                     (unsigned long long *)(slot + HMAP_STRIDE - 1), seq,
@@ -849,6 +854,18 @@ static GmresResult gmres(wb_ctx *c, int is_float, const void *b, void *x, double
         auto enqueue_step = [&](int k) {
             const bool cparts = apply_constrained(c, mode, vec(k), w, true);
             apply_precond(c, is_float, w, z, cparts);
+            if (arnoldi1_fits(is_float, k + 1, n)) {
+                const unsigned long long sq = ++c->hmap_seq;
+                double *slot = c->hmap_dev + (sq & 1) * HMAP_STRIDE;
+                const bool xc = cluster_copy(c, is_float);
+                launch_arnoldi1(is_float, V.p, ldv, k + 1, z, n, vec(k + 1),
+                                c->hbuf.as<double>(), c->stream, slot,
+                                (unsigned long long *)(slot + HMAP_STRIDE - 1), sq,
+                                xc ? c->hm_T.as<float>() : nullptr,
+                                xc ? c->hm_pos.as<int>() : nullptr);
+                c->hm_xc_for = xc ? vec(k + 1) : nullptr;
+                return sq;
+            }
             double *h1 = c->hred.as<double>(), *h2 = h1 + KMAX;
             launch_dot_partials(is_float, V.p, ldv, k + 1, z, n, c->P1.as<double>(), c->stream);
             launch_update_dot(is_float, V.p, ldv, k + 1, nullptr, z, n, c->P2.as<double>(),

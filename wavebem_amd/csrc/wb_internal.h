@@ -382,6 +382,16 @@ void launch_finalize(int is_float, int kcount, const double *h1, const double *h
                      size_t sH = 0, const int *active = nullptr, double *hmap = nullptr,
                      unsigned long long *hseq = nullptr, unsigned long long seq = 0,
                      float *xcl = nullptr, const int *pos = nullptr);
+#ifndef WB_ARNOLDI1_KB
+#define WB_ARNOLDI1_KB 160
+#endif
+constexpr int ARNOLDI1_MAX_N = 4096;
+constexpr size_t ARNOLDI1_BYTES = WB_ARNOLDI1_KB * 1024;
+bool arnoldi1_fits(int is_float, int kcount, int n);
+void launch_arnoldi1(int is_float, const void *V, size_t ldv, int kcount, const void *z, int n,
+                     void *vout, double *hout, hipStream_t s, double *hmap,
+                     unsigned long long *hseq, unsigned long long seq, float *xcl,
+                     const int *pos);
 void launch_axpy_basis(int is_float, const void *V, size_t ldv, int kcount, const double *y,
                        void *x_acc, int x_is_float, int n, hipStream_t s, int batch = 1,
                        size_t sV = 0, size_t sY = 0, size_t sX = 0, const int *active = nullptr);

@@ -260,6 +260,77 @@ __global__ __launch_bounds__(KTHREADS) void k_finalize(int kcount, const double 
     }
 }
 
+// One Arnoldi step of a small problem in one workgroup: both passes, the norm, the new
+// basis vector and the publication (as k_dot_partials, k_update_dot twice and k_finalize, with
+// the same roundings of z; the sums of a dot are formed by one wavefront in a fixed order).
+// One launch in place of four, which cost about 5 us each whatever the size; the basis is
+// read four times through one CU, so only up to ARNOLDI1_BYTES of it (launch_arnoldi1).
+constexpr int A1_THREADS = 1024;
+
+template <typename T>
+__global__ __launch_bounds__(A1_THREADS) void k_arnoldi1(
+    const T *__restrict__ V, size_t ldv, int kcount, const T *__restrict__ z, int n,
+    T *__restrict__ vout, double *__restrict__ hout, double *__restrict__ hmap,
+    unsigned long long *__restrict__ hseq, unsigned long long seq, float *__restrict__ xcl,
+    const int *__restrict__ pos)
+{
+    __shared__ T zs[ARNOLDI1_MAX_N];
+    __shared__ double h[2][KMAX];
+    __shared__ double red[A1_THREADS / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int e = tid; e < n; e += A1_THREADS) zs[e] = z[e];
+    double nrm = 0.0;
+#pragma unroll
+    for (int pass = 0; pass < 2; ++pass) {
+        __syncthreads();
+        for (int k = wave; k < kcount; k += A1_THREADS / 64) {
+            const T *vk = V + (size_t)k * ldv;
+            double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+            int e = lane;
+            for (; e + 192 < n; e += 256) {
+                s0 += (double)vk[e] * (double)zs[e];
+                s1 += (double)vk[e + 64] * (double)zs[e + 64];
+                s2 += (double)vk[e + 128] * (double)zs[e + 128];
+                s3 += (double)vk[e + 192] * (double)zs[e + 192];
+            }
+            for (; e < n; e += 64) s0 += (double)vk[e] * (double)zs[e];
+            const double s = ksum((s0 + s1) + (s2 + s3));
+            if (lane == 0) h[pass][k] = s;
+        }
+        __syncthreads();
+        for (int e = tid; e < n; e += A1_THREADS) {
+            double a = (double)zs[e];
+            for (int k = 0; k < kcount; ++k) a -= h[pass][k] * (double)V[(size_t)k * ldv + e];
+            const T v = (T)a;
+            zs[e] = v;
+            if (pass == 1) nrm += (double)v * (double)v;
+        }
+    }
+    nrm = ksum(nrm);
+    if (lane == 0) red[wave] = nrm;
+    __syncthreads();
+    double t = 0.0;
+    for (int w = 0; w < A1_THREADS / 64; ++w) t += red[w];
+    const double nv = sqrt(t);
+    for (int k = tid; k <= kcount; k += A1_THREADS) {
+        const double hk = k < kcount ? h[0][k] + h[1][k] : nv;
+        hout[k] = hk;
+        hmap[k] = hk;
+    }
+    __threadfence_system();
+    __syncthreads();
+    if (tid == 0) __hip_atomic_store(hseq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    const double inv = nv > 0 ? 1.0 / nv : 0.0;
+    for (int e = tid; e < n; e += A1_THREADS) {
+        const T v = (T)((double)zs[e] * inv);
+        vout[e] = v;
+        if (xcl) {
+            const int ps = pos[e];
+            if (ps >= 0) xcl[ps] = (float)v;
+        }
+    }
+}
+
 // x += sum_i y_i v_i   (x may be double while V is float)
 template <typename T, typename TX>
 __global__ void k_axpy_basis(const T *__restrict__ V, size_t ldv, size_t sV, int kcount,
@@ -364,6 +435,30 @@ void launch_finalize(int is_float, int kcount, const double *h1, const double *h
         hipLaunchKernelGGL(k_finalize<double>, grid, dim3(KTHREADS), 0, s, kcount, h1, h2, sHin,
                            Pn, (const double *)z, sZ, n, (double *)vout, sV, hout, sH, active,
                            hmap, hseq, seq, (float *)nullptr, pos);
+}
+
+// Whether an Arnoldi step with kcount basis vectors goes to k_arnoldi1: the basis it reads
+// four times through one CU stays within ARNOLDI1_BYTES.  Steps of the FP32-IR solve, limits
+// of 40, 160 and 400 KB: 2.10, 2.08, 2.11 ms at 1,083 dofs (2.41 with four launches always),
+// 2.63, 2.58, 2.60 at 2,915 (2.81); FP64 at 2,915 2.15, 2.14, 2.21 (2.19).
+bool arnoldi1_fits(int is_float, int kcount, int n)
+{
+    return n <= ARNOLDI1_MAX_N && (size_t)kcount * n * (is_float ? 4 : 8) <= ARNOLDI1_BYTES;
+}
+
+void launch_arnoldi1(int is_float, const void *V, size_t ldv, int kcount, const void *z, int n,
+                     void *vout, double *hout, hipStream_t s, double *hmap,
+                     unsigned long long *hseq, unsigned long long seq, float *xcl,
+                     const int *pos)
+{
+    if (is_float)
+        hipLaunchKernelGGL(k_arnoldi1<float>, dim3(1), dim3(A1_THREADS), 0, s, (const float *)V,
+                           ldv, kcount, (const float *)z, n, (float *)vout, hout, hmap, hseq,
+                           seq, xcl, pos);
+    else
+        hipLaunchKernelGGL(k_arnoldi1<double>, dim3(1), dim3(A1_THREADS), 0, s,
+                           (const double *)V, ldv, kcount, (const double *)z, n, (double *)vout,
+                           hout, hmap, hseq, seq, (float *)nullptr, pos);
 }
 
 void launch_axpy_basis(int is_float, const void *V, size_t ldv, int kcount, const double *y,
