@@ -874,10 +874,15 @@ __global__ __launch_bounds__(256) void k_hm_sum_parts(int n, int nagg, int npart
 #ifndef WB_HM_WAVES
 #define WB_HM_WAVES 8192
 #endif
+// at most this many chunks: every chunk is a partial sum per row that k_hm_finish adds (12 us
+// for 128 of them at 1,083 dofs, 9 at 21k), and few clusters have few blocks to spread
+#ifndef WB_HM_CHUNKS
+#define WB_HM_CHUNKS 48
+#endif
 int hm_chunks(int ncl)
 {
     const int c = (WB_HM_WAVES + ncl - 1) / ncl;
-    return std::max(1, std::min(128, c));
+    return std::max(1, std::min(WB_HM_CHUNKS, c));
 }
 
 
