@@ -464,157 +464,198 @@ __global__ __launch_bounds__(64 * MW) void k_gemm_sel_d(
     }
 }
 
-// The hi + bf16 lo operator (FP64 vectors) with LDS-staged panels: the block's 128 rows x
-// HL_P columns of the selected hi (FP32) and lo (bf16) entries are staged with whole-row
-// loads (at 64 columns a wavefront reads 4 rows x 256 bytes of hi and 4 rows x 128 bytes of
-// lo per instruction), the panel's vector entries once per block with their signs, and
-// contracted on the FP64 matrix cores as in k_gemm_sel_d.  A staging
-// thread owns one 4-column group of the panel: gmask says whether its columns read G or H
-// (both, column by column, for a mixed group); the signs go to the vector operand.
-// LDS row strides of HL_U + 1 (hi, 16-byte units) and HL_U + 2 (lo, 8-byte units) put the
-// 16 rows of a fragment read in distinct banks.  At 61k, k = 8: 64-column panels, 2 blocks
-// per CU (61.5 KB of LDS each), 4.68 ms; 32 columns, 4 blocks per CU, 4.96 ms; 16 columns
-// 8.87 ms.
-#ifndef WB_MULTI_HL_PANEL
-#define WB_MULTI_HL_PANEL 64
-#endif
-constexpr int HL_P = WB_MULTI_HL_PANEL;  // columns per panel (a multiple of 16)
-constexpr int HL_U = HL_P / 4;      // 4-column groups per panel row
-constexpr int HL_SH = HL_U + 1;     // hi row stride (16-byte units)
-constexpr int HL_SL = HL_U + 2;     // lo row stride (8-byte units)
+// The hi + bf16 lo operator (FP64 vectors): every wavefront contracts its own 32 rows by
+// panels of HL_P columns and shares nothing with the others of its block, so there is no
+// barrier in the kernel.  A panel's selected hi (FP32) and lo (bf16) entries go from memory
+// straight into the wavefront's LDS (16 bytes per lane; no registers and no LDS write
+// instructions on the way): 8 loads of 4 rows x 256 bytes of hi, 4 of 8 rows x 128 bytes of
+// lo.  One panel is always on its way: the panel that has arrived is read into registers as
+// raw fragments (48 registers), the next one is requested into the same LDS, and only then
+// is the current one contracted on the FP64 matrix cores as in k_gemm_sel_d.
+//
+// The lanes of such a load fill consecutive LDS units, so rows cannot be padded; instead
+// lane -> column group is permuted inside each row (unit = group ^ row), which puts the 16
+// rows of a fragment read in distinct banks.  A panel that mixes G and H columns, or is cut
+// by the end of the columns, is staged through registers, column by column, in the same
+// layout.
+//
+// Bound: memory.  At 61k unknowns and k = 8 (22.4 GB of operator) 3.79 ms, 5.9 TB/s; the
+// block-wide panels staged through registers and two barriers that this replaces took
+// 4.84 ms (2 blocks per CU), and this kernel 4.35 ms with a grid of 3.1 rounds of resident
+// blocks instead of whole rounds (multi_chunks).
+//
+// X is read up to the end of the last panel: every column of X has ld readable entries, 16
+// bytes aligned (what lies past the columns is not used).
+constexpr int HL_P = 64;          // columns per panel
+constexpr int HL_U = HL_P / 4;    // 4-column groups per panel
+constexpr int HL_R = 16 * RT;     // rows per wavefront
+constexpr int HL_WAVES = 3;       // blocks per CU that 48 KB of LDS per block allow
 
-#ifndef WB_MULTI_HL_WAVES
-#define WB_MULTI_HL_WAVES 2  // wavefronts per SIMD the hi + lo kernel is built for (the
-                             // blocks per CU its LDS allows)
-#endif
+#define WB_GLOBAL_AS __attribute__((address_space(1)))
+#define WB_LDS_AS __attribute__((address_space(3)))
 
-__global__ __launch_bounds__(64 * MW, WB_MULTI_HL_WAVES) void k_gemm_hl_lds(
+__device__ __forceinline__ int clamped_row(int slot, const int *rows, int n_rows)
+{
+    slot = min(slot, n_rows - 1);
+    return rows ? rows[slot] : slot;
+}
+
+// 16 bytes per lane from src (per lane) to dst + 16 * lane (dst the same in all lanes);
+// non-temporal
+__device__ __forceinline__ void load_to_lds16(const void *src, void *dst)
+{
+    __builtin_amdgcn_global_load_lds((WB_GLOBAL_AS void *)(uintptr_t)src,
+                                     (WB_LDS_AS void *)dst, 16, 0, 2);
+}
+
+__global__ __launch_bounds__(64 * MW, HL_WAVES) void k_gemm_hl(
     const float *__restrict__ G, const float *__restrict__ H, const uint16_t *__restrict__ Glo,
     const uint16_t *__restrict__ Hlo, size_t ld, int n, const uint8_t *__restrict__ gmask,
     int flip, double s_sel, double s_uns, int k, const double *__restrict__ X, size_t ldx,
     const int *__restrict__ rows, int n_rows, int cols_per_chunk, double *__restrict__ part)
 {
-    __shared__ fvec4 tile_h[RPB * HL_SH];
-    __shared__ uvec4 tile_l[RPB * HL_SL];
-    // the panel's vector entries, signs applied: [v][column] (loaded once per block)
-    __shared__ double xtile[WB_MULTI_MAX * (HL_P + 1)];
+    __shared__ fvec4 tile_h[MW * HL_R * HL_U];
+    __shared__ uvec4 tile_l[MW * HL_R * HL_U];
     const int c0 = blockIdx.y * cols_per_chunk, c1 = min(n, c0 + cols_per_chunk);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int brow = blockIdx.x * RPB;
-    constexpr int SR = 64 * MW / HL_U;  // rows per staging pass
-    constexpr int SJ = RPB / SR;        // staging passes
-    const int su = tid % HL_U, sr = tid / HL_U;
-    // staged rows as 32-bit indices (their 64-bit offsets are formed at each load, which
-    // keeps 4 registers free)
-    int srow[SJ];
-#pragma unroll
-    for (int j = 0; j < SJ; ++j) srow[j] = tile_row(brow + sr + SR * j, rows, n_rows);
-    const int i = lane & 15, q = lane >> 4;
-    const int v = lane & 15;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int base = blockIdx.x * RPB + wave * HL_R;
+    fvec4 *th = tile_h + wave * (HL_R * HL_U);
+    uvec4 *tl = tile_l + wave * (HL_R * HL_U);
+    // the wavefront's rows, kept in LDS: registers decide how many wavefronts fit
+    __shared__ int tile_r[MW * HL_R];
+    int *tr = tile_r + wave * HL_R;
+    if (lane < HL_R) tr[lane] = clamped_row(base + lane, rows, n_rows);
+    constexpr int JH = HL_R / 4, JL = HL_R / 8;  // loads of a panel: hi 4 rows, lo 8 rows each
+    const int i = lane & 15, q = lane >> 4, v = lane & 15;
     const bool vok = v < k;
-    const unsigned fm = flip ? 0xfu : 0u;
+    const unsigned fm = flip ? 0x0f0f0f0fu : 0u;
+    const double *xv = X + (size_t)(vok ? v : 0) * ldx + 4 * q;
     dvec4 c[RT];
 #pragma unroll
     for (int t = 0; t < RT; ++t) c[t] = dvec4{0.0, 0.0, 0.0, 0.0};
-    fvec4 sh[SJ];
-    uvec4 sl[SJ];
-    // stage: group su of the panel at pc for rows sr + SR j
-    auto load_panel = [&](int pc) {
-        // an empty asm that "changes" the rows keeps their 64-bit offsets from being
-        // hoisted out of the panel loop into registers
+    // byte u of word w: group 4 w + u of the panel at pc, bit e set where column e reads H
+    // (mn: the panel after it, read a panel early)
+    unsigned mk[4], mn[4];
+    auto masks = [&](int pc) {
+        const int g0 = min(pc, (int)ld - HL_P) >> 2;
 #pragma unroll
-        for (int j = 0; j < SJ; ++j) asm volatile("" : "+v"(srow[j]));
-        const int scol = pc + 4 * su;
-        const fvec4 z4 = {0.f, 0.f, 0.f, 0.f};
-        const uvec4 zl = {0, 0, 0, 0};
-        if (scol < c1) {
-            const unsigned m = (unsigned)gmask[scol >> 2] ^ fm;  // bit e: column e reads H
-            if (m == 0u || m == 0xfu) {
-                const float *M = m ? H : G;
-                const uint16_t *L = m ? Hlo : Glo;
+        for (int w = 0; w < 4; ++w) mn[w] = *(const unsigned *)(gmask + g0 + 4 * w) ^ fm;
+    };
+    dvec2 xn[2 * HL_U / 4];
+    auto stage = [&](int pc) {
+        unsigned any = 0u, all = 0x0f0f0f0fu;
 #pragma unroll
-                for (int j = 0; j < SJ; ++j) {
-                    sh[j] = __builtin_nontemporal_load((const fvec4 *)(M + (size_t)srow[j] * ld + scol));
-                    sl[j] = __builtin_nontemporal_load((const uvec4 *)(L + (size_t)srow[j] * ld + scol));
-                }
-            } else {
+        for (int w = 0; w < 4; ++w) {
+            mk[w] = mn[w];
+            any |= mk[w];
+            all &= mk[w];
+        }
+        if (pc + HL_P <= c1 && (any == 0u || all == 0x0f0f0f0fu)) {
+            const float *M = (any ? H : G) + pc;
+            const uint16_t *L = (any ? Hlo : Glo) + pc;
+            // (an empty asm that "changes" the lane keeps the rows from being hoisted out of
+            // the panel loop into registers)
+            int la = lane;
+            asm volatile("" : "+v"(la));
+            int rh[JH], rl[JL];
 #pragma unroll
-                for (int j = 0; j < SJ; ++j) {
-                    const fvec4 g = *(const fvec4 *)(G + (size_t)srow[j] * ld + scol);
-                    const fvec4 h = *(const fvec4 *)(H + (size_t)srow[j] * ld + scol);
-                    const uvec4 gl = *(const uvec4 *)(Glo + (size_t)srow[j] * ld + scol);
-                    const uvec4 hl = *(const uvec4 *)(Hlo + (size_t)srow[j] * ld + scol);
+            for (int j = 0; j < JH; ++j) rh[j] = tr[4 * j + (la >> 4)];
+#pragma unroll
+            for (int j = 0; j < JL; ++j) rl[j] = tr[8 * j + (la >> 3)];
+#pragma unroll
+            for (int j = 0; j < JH; ++j) asm volatile("" : "+v"(rh[j]));
+#pragma unroll
+            for (int j = 0; j < JL; ++j) asm volatile("" : "+v"(rl[j]));
+#pragma unroll
+            for (int j = 0; j < JH; ++j) {
+                const int g = (la & 15) ^ ((4 * j + (la >> 4)) & 15);
+                load_to_lds16(M + (size_t)rh[j] * ld + 4 * g, th + 64 * j);
+            }
+#pragma unroll
+            for (int j = 0; j < JL; ++j) {
+                const int g = (la & 7) ^ (la >> 3);
+                load_to_lds16(L + (size_t)rl[j] * ld + 8 * g, tl + 128 * j);
+            }
+        } else {
+#pragma unroll 1
+            for (int j = 0; j < JH; ++j) {
+                const int r = 4 * j + (lane >> 4), g = (lane & 15) ^ (r & 15);
+                const int col = pc + 4 * g;
+                const size_t o = (size_t)tr[r] * ld + col;
+                fvec4 hv = {0.f, 0.f, 0.f, 0.f};
+                uvec4 lv = {0, 0, 0, 0};
+                if (col < c1) {
+                    const unsigned m = (unsigned)gmask[col >> 2] ^ (fm & 0xfu);
+                    const fvec4 gh = *(const fvec4 *)(G + o), hh = *(const fvec4 *)(H + o);
+                    const uvec4 gl = *(const uvec4 *)(Glo + o), hl = *(const uvec4 *)(Hlo + o);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const bool he = (m >> e) & 1u;
-                        sh[j][e] = he ? h[e] : g[e];
-                        sl[j][e] = he ? hl[e] : gl[e];
+                        hv[e] = he ? hh[e] : gh[e];
+                        lv[e] = he ? hl[e] : gl[e];
                     }
                 }
+                th[r * HL_U + (lane & 15)] = hv;
+                tl[2 * (r * (HL_U / 2) + ((g >> 1) ^ (r & 7))) + (g & 1)] = lv;
             }
-        } else {
+        }
+        masks(pc + HL_P);
+        // this lane's vector entries: columns pc + 16 u + 4 q .. + 3
 #pragma unroll
-            for (int j = 0; j < SJ; ++j) {
-                sh[j] = z4;
-                sl[j] = zl;
-            }
+        for (int u = 0; u < HL_U / 4; ++u) {
+            xn[2 * u] = *(const dvec2 *)(xv + pc + 16 * u);
+            xn[2 * u + 1] = *(const dvec2 *)(xv + pc + 16 * u + 2);
         }
     };
+    masks(c0);
+    if (c0 < c1) stage(c0);
     for (int cb = c0; cb < c1; cb += HL_P) {
-        load_panel(cb);
-        constexpr int XE = (WB_MULTI_MAX * HL_P + 64 * MW - 1) / (64 * MW);
-        double sx[XE];
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the panel and its vector entries are here
+        double b[HL_U / 4][4];
 #pragma unroll
-        for (int j = 0; j < XE; ++j) {
-            const int t = tid + 64 * MW * j, vv = t / HL_P, cc = cb + t % HL_P;
-            double xv = 0.0;
-            if (vv < k && cc < c1) {
-                const unsigned m = (unsigned)gmask[cc >> 2] ^ fm;
-                xv = X[(size_t)vv * ldx + cc] * (((m >> (cc & 3)) & 1u) ? s_sel : s_uns);
+        for (int u = 0; u < HL_U / 4; ++u) {
+            const unsigned m = mk[u] >> (8 * q);
+            const bool in = vok && cb + 16 * u + 4 * q < c1;  // zero past the chunk
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const double x = xn[2 * u + (e >> 1)][e & 1] * (((m >> e) & 1u) ? s_sel : s_uns);
+                b[u][e] = in ? x : 0.0;
+                // (formed here, so that xn is free for the next panel's entries)
+                asm volatile("" : "+v"(b[u][e]));
             }
-            sx[j] = xv;
         }
-        __syncthreads();  // the previous panel's fragments have been read
+        fvec4 fh[HL_U / 4][RT];
+        uvec4 fl[HL_U / 4][RT];
 #pragma unroll
-        for (int j = 0; j < SJ; ++j) {
-            tile_h[(sr + SR * j) * HL_SH + su] = sh[j];
-            tile_l[(sr + SR * j) * HL_SL + su] = sl[j];
-        }
-#pragma unroll
-        for (int j = 0; j < XE; ++j) {
-            const int t = tid + 64 * MW * j;
-            if (t < WB_MULTI_MAX * HL_P) xtile[(t / HL_P) * (HL_P + 1) + t % HL_P] = sx[j];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < HL_P / 16; ++u) {
-            // this lane's 4 columns cb + 16 u + 4 q .. + 3, signs applied (zero past the chunk)
-            double b[4] = {0.0, 0.0, 0.0, 0.0};
-            if (vok) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) b[e] = xtile[v * (HL_P + 1) + 16 * u + 4 * q + e];
-            }
-            double a[RT][4];
+        for (int u = 0; u < HL_U / 4; ++u)
 #pragma unroll
             for (int t = 0; t < RT; ++t) {
-                const int r = wave * 16 * RT + 16 * t + i;
-                const fvec4 h = tile_h[r * HL_SH + 4 * u + q];
-                const uvec4 l = tile_l[r * HL_SL + 4 * u + q];
+                const int r = 16 * t + i, g = 4 * u + q;
+                fh[u][t] = th[r * HL_U + (g ^ i)];
+                fl[u][t] = tl[2 * (r * (HL_U / 2) + ((g >> 1) ^ (i & 7))) + (g & 1)];
+            }
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the panel is read, its LDS is free
+        if (cb + HL_P < c1) stage(cb + HL_P);
+#pragma unroll
+        for (int u = 0; u < HL_U / 4; ++u) {
+            double a[RT][4];
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    a[t][e] = (double)h[e] + (double)__uint_as_float((uint32_t)l[e] << 16);
-            }
+                    a[t][e] = (double)fh[u][t][e] +
+                              (double)__uint_as_float((uint32_t)fl[u][t][e] << 16);
 #pragma unroll
             for (int s2 = 0; s2 < 4; ++s2)
 #pragma unroll
                 for (int t = 0; t < RT; ++t)
-                    c[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t][s2], b[s2], c[t], 0, 0, 0);
+                    c[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t][s2], b[u][s2], c[t], 0, 0, 0);
         }
     }
     // FP64 result layout: D[i][j] in lane j + 16 (i % 4), register i / 4
     if (vok) {
         double *pp = part + ((size_t)blockIdx.y * k + v) * n_rows;
-        const int base = brow + wave * 16 * RT;
 #pragma unroll
         for (int t = 0; t < RT; ++t)
 #pragma unroll
@@ -643,22 +684,25 @@ __global__ void k_multi_reduce(const double *__restrict__ part, int n_chunks, in
 
 }  // namespace
 
-// Column chunks of the batched product.  The matrix-core kernels of modes 0-2 take about
-// 8k wavefronts whatever n is.  The FP16 kernel (mode 3) streams the operator at close to
-// the memory rate, so its grid is sized in whole rounds of resident blocks: the chunk count
-// (1..16) whose block count comes closest to a multiple of what the device holds at once,
-// the smaller count on ties.
+// Column chunks of the batched product.  The matrix-core kernels of modes 0 and 1 take about
+// 8k wavefronts whatever n is.  The hi + lo and the FP16 kernels (modes 2 and 3) stream the
+// operator at close to the memory rate, so their grids are sized in whole rounds of resident
+// blocks: the chunk count (1..16) whose block count comes closest to a multiple of what the
+// device holds at once, the smaller count on ties (at 61k 8 chunks, 5 rounds, instead of 5
+// chunks, 3.1 rounds: 4.35 -> 3.79 ms).
 int multi_chunks(int mode, int n_rows, int n_groups)
 {
     // the resident-block count is cached (a failed query stays 0 and selects the rule of the
     // other modes below: a grid shape only, the sums are the same), so the workspace sizing
     // and the launch always agree
-    const int cap = mode == 3 ? resident_blocks(reinterpret_cast<const void *>(&k_gemm_h16),
-                                                64 * MW)
-                              : 0;
-    if (mode == 3 && cap > 0) {
+    const void *kern = mode == 3   ? reinterpret_cast<const void *>(&k_gemm_h16)
+                       : mode == 2 ? reinterpret_cast<const void *>(&k_gemm_hl)
+                                   : nullptr;
+    const int cap = kern ? resident_blocks(kern, 64 * MW) : 0;
+    if (cap > 0) {
         const long long blocks = (n_rows + RPB - 1) / RPB;
-        const int steps = (4 * n_groups + HP16 - 1) / HP16;
+        const int panel = mode == 3 ? HP16 : HL_P;
+        const int steps = (4 * n_groups + panel - 1) / panel;
         int best = 1;
         double best_fill = 0.0;
         for (int c = 1; c <= 16 && c <= std::max(1, steps); ++c) {
@@ -710,7 +754,7 @@ void launch_gemv_sel_multi(int mode, const void *G, const void *H, const void *G
         // chunks of whole HL_P-column panels (chunks past the columns write zero sums)
         const int n = 4 * n_groups;
         const int cpc = ((n + chunks - 1) / chunks + HL_P - 1) / HL_P * HL_P;
-        hipLaunchKernelGGL(k_gemm_hl_lds, grid, block, 0, s, (const float *)G, (const float *)H,
+        hipLaunchKernelGGL(k_gemm_hl, grid, block, 0, s, (const float *)G, (const float *)H,
                            (const uint16_t *)Glo, (const uint16_t *)Hlo, ld, n, gmask, flip,
                            s_sel, s_unsel, k, (const double *)X, ldx, rows, n_rows, cpc, part);
     }
