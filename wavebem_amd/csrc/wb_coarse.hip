@@ -299,49 +299,59 @@ __global__ __launch_bounds__(256) void k_coarse_residual(int n, int nc, const T 
             (T)((double)X[(size_t)v * ldx + i] - (((qs[0][rl] + qs[1][rl]) + qs[2][rl]) + qs[3][rl]));
 }
 
-// The block-Jacobi apply of one vector with the coarse residual formed in the same
-// workgroup (blocks of bs <= 64 rows, 256 threads): t = x - W C for the block's rows, four
-// quarter sums per row as in k_coarse_residual; z_a = (Aci C)_a for the aggregates the rows
-// touch, one wavefront each; then y = B^-1 t + z, the columns of B^-1 split over the four
-// wavefronts and the partial products added in wavefront order.  x and y may alias: every
-// row is read and written by its own workgroup only, the read before the write.
-#ifndef WB_BJC_WAVES
-#define WB_BJC_WAVES 4
-#endif
-constexpr int BJC_W = WB_BJC_WAVES;  // wavefronts per 64-row block
+// The block-Jacobi apply with the coarse residual formed in the same workgroup (blocks of
+// bs <= 64 rows, 256 threads), for KV of the k vectors (group blockIdx.y): t = x - W C for
+// the block's rows, four quarter sums per row; z_a = (Aci C)_a for the aggregates the rows
+// touch, one wavefront per sum; then y = B^-1 t + z, the columns of B^-1 split over the four
+// wavefronts and the partial products added in wavefront order.  W and B^-1 are read once
+// for the KV vectors.  x and y may alias: every row is read and written by its own workgroup
+// only, the read before the write.
+//
+// Bound: the reads of W (31 MB in FP32 at 61k and 128 aggregates) and, with KV = 8, the FP64
+// sums.  Eight FP32 vectors at 61k: 19.5 us; the residual and the blocks in kernels of their
+// own, each reading its matrix once per vector, 38.5 + 33.7 us.
+constexpr int BJC_W = 4;  // wavefronts per 64-row block
 
-template <typename T>
+template <typename T, int KV>
 __global__ __launch_bounds__(64 * BJC_W) void k_bj_coarse(int n, int bs, const T *__restrict__ binv,
-                                                   const T *x, T *y, const T *__restrict__ WT,
+                                                   const T *x, T *y, int k, size_t ldx,
+                                                   const T *__restrict__ WT,
                                                    size_t ldw, const double *__restrict__ C,
                                                    const T *__restrict__ Aci, int nc, int agg,
                                                    const double *__restrict__ Cpart)
 {
-    __shared__ double cs[CS_MAX];
-    __shared__ double qs[BJC_W][64];
-    __shared__ T ts[64];
-    __shared__ T ps[BJC_W][64];
-    __shared__ double zs[4];
+    __shared__ double cs[CS_MAX][KV];
+    __shared__ double qs[BJC_W][KV][64];
+    __shared__ T ts[64][KV];
+    __shared__ T ps[BJC_W][KV][64];
+    __shared__ double zs[4][KV];
     const int tid = threadIdx.x, rl = tid & 63, w = tid >> 6;
     const int base = blockIdx.x * bs, m = min(bs, n - base);
-    for (int b = tid; b < nc; b += 64 * BJC_W) {
-        double v;
-        if (Cpart) {
-            // aggregate b from the partial sums of the 64-row blocks it overlaps, in order
+    const int v0 = blockIdx.y * KV, kv = min(KV, k - v0);
+    x += (size_t)v0 * ldx;
+    y += (size_t)v0 * ldx;
+    if (KV == 1 && Cpart) {
+        // aggregate b from the partial sums of the 64-row blocks it overlaps, in order
+        for (int b = tid; b < nc; b += 64 * BJC_W) {
             const int r0 = b * agg, r1 = min(n, (b + 1) * agg);
-            v = 0.0;
+            double v = 0.0;
             for (int blk = r0 / 64; blk <= (r1 - 1) / 64; ++blk)
                 v += Cpart[2 * blk + (b - (blk * 64) / agg)];
-        } else {
-            v = C[b];
+            cs[b][0] = v;
         }
-        cs[b] = v;
+    } else {
+#pragma unroll
+        for (int v = 0; v < KV; ++v)
+            for (int b = tid; b < nc; b += 64 * BJC_W)
+                cs[b][v] = v < kv ? C[(size_t)(v0 + v) * CS_MAX + b] : 0.0;
     }
     __syncthreads();
     const int i = base + rl;
     const int b0 = w * nc / BJC_W, b1 = (w + 1) * nc / BJC_W;
     // loads in batches of 16 (independent, so one wait per batch), two accumulators
-    double a0 = 0.0, a1 = 0.0;
+    double a0[KV], a1[KV];
+#pragma unroll
+    for (int v = 0; v < KV; ++v) a0[v] = a1[v] = 0.0;
     if (rl < m) {
         int b = b0;
         for (; b + 16 <= b1; b += 16) {
@@ -349,34 +359,44 @@ __global__ __launch_bounds__(64 * BJC_W) void k_bj_coarse(int n, int bs, const T
 #pragma unroll
             for (int u = 0; u < 16; ++u) wv[u] = WT[(size_t)(b + u) * ldw + i];
 #pragma unroll
-            for (int u = 0; u < 16; u += 2) {
-                a0 = fma((double)wv[u], cs[b + u], a0);
-                a1 = fma((double)wv[u + 1], cs[b + u + 1], a1);
-            }
+            for (int u = 0; u < 16; u += 2)
+#pragma unroll
+                for (int v = 0; v < KV; ++v) {
+                    a0[v] = fma((double)wv[u], cs[b + u][v], a0[v]);
+                    a1[v] = fma((double)wv[u + 1], cs[b + u + 1][v], a1[v]);
+                }
         }
-        for (; b < b1; ++b) a0 = fma((double)WT[(size_t)b * ldw + i], cs[b], a0);
+        for (; b < b1; ++b) {
+            const double wb = (double)WT[(size_t)b * ldw + i];
+#pragma unroll
+            for (int v = 0; v < KV; ++v) a0[v] = fma(wb, cs[b][v], a0[v]);
+        }
     }
-    qs[w][rl] = a0 + a1;
+#pragma unroll
+    for (int v = 0; v < KV; ++v) qs[w][v][rl] = a0[v] + a1[v];
     const int ag0 = base / agg, na = (base + m - 1) / agg - ag0 + 1;
-    if (w < na) {
-        const int a = ag0 + w;
+    for (int t = w; t < na * KV; t += BJC_W) {
+        const int a = t / KV, v = t % KV;
         double p = 0.0;
 #pragma unroll 3
-        for (int bb = rl; bb < nc; bb += 64) p += (double)Aci[(size_t)a * nc + bb] * cs[bb];
+        for (int bb = rl; bb < nc; bb += 64)
+            p += (double)Aci[(size_t)(ag0 + a) * nc + bb] * cs[bb][v];
         p = cs_wave_sum(p);
-        if (rl == 0) zs[w] = p;
+        if (rl == 0) zs[a][v] = p;
     }
     __syncthreads();
-    if (w == 0) {
-        double q = qs[0][rl];
+    for (int v = w; v < KV; v += BJC_W) {
+        double q = qs[0][v][rl];
 #pragma unroll
-        for (int u = 1; u < BJC_W; ++u) q += qs[u][rl];
-        ts[rl] = rl < m ? (T)((double)x[i] - q) : (T)0;
+        for (int u = 1; u < BJC_W; ++u) q += qs[u][v][rl];
+        ts[rl][v] = rl < m && v < kv ? (T)((double)x[(size_t)v * ldx + i] - q) : (T)0;
     }
     __syncthreads();
     const int c0 = w * bs / BJC_W, c1 = min(m, (w + 1) * bs / BJC_W);
     const T *B = binv + (size_t)blockIdx.x * bs * bs;
-    T acc = 0;
+    T acc[KV];
+#pragma unroll
+    for (int v = 0; v < KV; ++v) acc[v] = 0;
     if (rl < m) {
         int c = c0;
         constexpr int CB = 64 / BJC_W;  // columns per wavefront at bs = 64, loaded together
@@ -385,18 +405,43 @@ __global__ __launch_bounds__(64 * BJC_W) void k_bj_coarse(int n, int bs, const T
 #pragma unroll
             for (int u = 0; u < CB; ++u) bv[u] = B[(size_t)(c + u) * bs + rl];
 #pragma unroll
-            for (int u = 0; u < CB; ++u) acc += bv[u] * ts[c + u];
-        }
-        for (; c < c1; ++c) acc += B[(size_t)c * bs + rl] * ts[c];
-    }
-    ps[w][rl] = acc;
-    __syncthreads();
-    if (w == 0 && rl < m) {
-        T p = ps[0][rl];
+            for (int u = 0; u < CB; ++u)
 #pragma unroll
-        for (int u = 1; u < BJC_W; ++u) p += ps[u][rl];
-        y[i] = (T)((double)p + zs[i / agg - ag0]);
+                for (int v = 0; v < KV; ++v) acc[v] += bv[u] * ts[c + u][v];
+        }
+        for (; c < c1; ++c) {
+            const T bc = B[(size_t)c * bs + rl];
+#pragma unroll
+            for (int v = 0; v < KV; ++v) acc[v] += bc * ts[c][v];
+        }
     }
+#pragma unroll
+    for (int v = 0; v < KV; ++v) ps[w][v][rl] = acc[v];
+    __syncthreads();
+    for (int v = w; v < kv; v += BJC_W)
+        if (rl < m) {
+            T p = ps[0][v][rl];
+#pragma unroll
+            for (int u = 1; u < BJC_W; ++u) p += ps[u][v][rl];
+            y[(size_t)v * ldx + i] = (T)((double)p + zs[i / agg - ag0][v]);
+        }
+}
+
+template <typename T>
+void bj_coarse(int n, int bs, const void *binv, const void *x, void *y, int k, size_t ldx,
+               const void *WT, size_t ldw, const double *C, const void *Aci, int nc, int agg,
+               const double *Cpart, hipStream_t s)
+{
+    const int nb = (n + bs - 1) / bs;
+    auto go = [&](auto kern, int kv) {
+        hipLaunchKernelGGL(kern, dim3(nb, (k + kv - 1) / kv), dim3(64 * BJC_W), 0, s, n, bs,
+                           (const T *)binv, (const T *)x, (T *)y, k, ldx, (const T *)WT, ldw, C,
+                           (const T *)Aci, nc, agg, Cpart);
+    };
+    // more vectors per workgroup read W and B^-1 less often
+    if (k == 1) go(k_bj_coarse<T, 1>, 1);
+    else if (k <= 4) go(k_bj_coarse<T, 4>, 4);
+    else go(k_bj_coarse<T, 8>, 8);
 }
 
 }  // namespace
@@ -478,18 +523,11 @@ void launch_coarse_restrict(int is_float, int n, int agg, int nc, const void *X,
 bool bj_coarse_fits(int bs, int agg, int nc) { return bs >= 4 && bs <= 64 && agg >= bs && nc <= CS_MAX; }
 
 void launch_bj_coarse(int is_float, int n, int bs, const void *binv, const void *x, void *y,
-                      const void *WT, size_t ldw, const double *C, const void *Aci, int nc,
-                      int agg, hipStream_t s, const double *Cpart)
+                      int k, size_t ldx, const void *WT, size_t ldw, const double *C,
+                      const void *Aci, int nc, int agg, hipStream_t s, const double *Cpart)
 {
-    const int nb = (n + bs - 1) / bs;
-    if (is_float)
-        hipLaunchKernelGGL(k_bj_coarse<float>, dim3(nb), dim3(64 * BJC_W), 0, s, n, bs,
-                           (const float *)binv, (const float *)x, (float *)y, (const float *)WT,
-                           ldw, C, (const float *)Aci, nc, agg, Cpart);
-    else
-        hipLaunchKernelGGL(k_bj_coarse<double>, dim3(nb), dim3(64 * BJC_W), 0, s, n, bs,
-                           (const double *)binv, (const double *)x, (double *)y,
-                           (const double *)WT, ldw, C, (const double *)Aci, nc, agg, Cpart);
+    if (is_float) bj_coarse<float>(n, bs, binv, x, y, k, ldx, WT, ldw, C, Aci, nc, agg, Cpart, s);
+    else bj_coarse<double>(n, bs, binv, x, y, k, ldx, WT, ldw, C, Aci, nc, agg, Cpart, s);
 }
 
 }  // namespace wb

@@ -574,12 +574,11 @@ static void block_precond(wb_ctx *c, int is_float, int k, const void *x, void *y
                           c->cs_C.as<double>(), c->cs_T.p, k, c->stream);
         launch_block_jacobi_apply(0, c->n, c->pc_bs, binv, c->cs_T.p, y, k, c->vlen, c->stream,
                                   1, c->cs_C.as<double>(), c->cs_Aci.p, c->cs_nc, c->cs_agg);
-    } else if (c->cs_on && !c->op_transpose && k == 1 &&
-               bj_coarse_fits(c->pc_bs, c->cs_agg, c->cs_nc)) {
+    } else if (c->cs_on && !c->op_transpose && bj_coarse_fits(c->pc_bs, c->cs_agg, c->cs_nc)) {
         if (!cparts)
             launch_coarse_restrict(is_float, c->n, c->cs_agg, c->cs_nc, x, c->vlen,
-                                   c->cs_C.as<double>(), 1, c->stream);
-        launch_bj_coarse(is_float, c->n, c->pc_bs, binv, x, y,
+                                   c->cs_C.as<double>(), k, c->stream);
+        launch_bj_coarse(is_float, c->n, c->pc_bs, binv, x, y, k, c->vlen,
                          is_float ? c->cs_WT32.p : c->cs_WT.p, c->vlen, c->cs_C.as<double>(),
                          is_float ? c->cs_Aci32.p : c->cs_Aci.p, c->cs_nc, c->cs_agg,
                          c->stream, cparts ? c->cs_Cpart.as<double>() : nullptr);

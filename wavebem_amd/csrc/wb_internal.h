@@ -305,14 +305,14 @@ constexpr int CS_MAX = 192, CS_MAX64 = 128;
 // C = P^T x alone (k vectors)
 void launch_coarse_restrict(int is_float, int n, int agg, int nc, const void *X, size_t ldx,
                             double *C, int k, hipStream_t s);
-// One vector: y = B^-1 (x - W C) + P Aci C in one kernel (x and y may alias); usable when
-// bj_coarse_fits(bs, agg, nc)
-// bj_coarse_fits(bs, agg, nc); with Cpart (see launch_hm_gemv), C = P^T x is summed from
-// those block partials instead of read from C
+// y_v = B^-1 (x_v - W C[v]) + P Aci C[v] for k vectors (column stride ldx) in one kernel (x
+// and y may alias); usable when bj_coarse_fits(bs, agg, nc).  With Cpart (one vector, see
+// launch_hm_gemv), C = P^T x is summed from those block partials instead of read from C
 bool bj_coarse_fits(int bs, int agg, int nc);
 void launch_bj_coarse(int is_float, int n, int bs, const void *binv, const void *x, void *y,
-                      const void *WT, size_t ldw, const double *C, const void *Aci, int nc,
-                      int agg, hipStream_t s, const double *Cpart = nullptr);
+                      int k, size_t ldx, const void *WT, size_t ldw, const double *C,
+                      const void *Aci, int nc, int agg, hipStream_t s,
+                      const double *Cpart = nullptr);
 size_t coarse_invert_lds_bytes(int nc);
 void launch_coarse_build(int n, int agg, int nc, const void *G, const void *H, int precision,
                          size_t ld, const void *A16, const float *rs16, const double *alpha,
