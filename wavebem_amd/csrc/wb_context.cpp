@@ -867,12 +867,10 @@ static GmresResult gmres(wb_ctx *c, int is_float, const void *b, void *x, double
             }
             double *h1 = c->hred.as<double>(), *h2 = h1 + KMAX;
             launch_dot_partials(is_float, V.p, ldv, k + 1, z, n, c->P1.as<double>(), c->stream);
-            launch_update_dot(is_float, V.p, ldv, k + 1, nullptr, z, n, c->P2.as<double>(),
-                              nullptr, 0, c->stream, 1, 0, 0, 0, nullptr, c->P1.as<double>(),
-                              h1);
-            launch_update_dot(is_float, V.p, ldv, k + 1, nullptr, z, n, nullptr,
-                              c->Pn.as<double>(), 1, c->stream, 1, 0, 0, 0, nullptr,
-                              c->P2.as<double>(), h2);
+            launch_update_dot(is_float, V.p, ldv, k + 1, z, n, c->P1.as<double>(), h1,
+                              c->P2.as<double>(), nullptr, c->stream);
+            launch_update_dot(is_float, V.p, ldv, k + 1, z, n, c->P2.as<double>(), h2, nullptr,
+                              c->Pn.as<double>(), c->stream);
             const unsigned long long sq = ++c->hmap_seq;
             finalize_publish(c, is_float, k + 1, h1, h2, z, n, vec(k + 1), sq);
             return sq;
@@ -1451,12 +1449,11 @@ static std::vector<int> gmres_multi(wb_ctx *c, int is_float, int k, const void *
             double *h1 = M.hred.as<double>(), *h2 = h1 + KMAX;
             launch_dot_partials(is_float, V.p, vl, kc, Z, n, M.P1.as<double>(), c->stream, k, sV,
                                 vl, M.act.as<int>());
-            launch_reduce_parts(kc, M.P1.as<double>(), n, h1, c->stream, k, sR, M.act.as<int>());
-            launch_update_dot(is_float, V.p, vl, kc, h1, Z, n, M.P2.as<double>(), nullptr, 0,
-                              c->stream, k, sV, vl, sR, M.act.as<int>());
-            launch_reduce_parts(kc, M.P2.as<double>(), n, h2, c->stream, k, sR, M.act.as<int>());
-            launch_update_dot(is_float, V.p, vl, kc, h2, Z, n, nullptr, M.Pn.as<double>(), 1,
-                              c->stream, k, sV, vl, sR, M.act.as<int>());
+            launch_update_dot(is_float, V.p, vl, kc, Z, n, M.P1.as<double>(), h1,
+                              M.P2.as<double>(), nullptr, c->stream, k, sV, vl, sR,
+                              M.act.as<int>());
+            launch_update_dot(is_float, V.p, vl, kc, Z, n, M.P2.as<double>(), h2, nullptr,
+                              M.Pn.as<double>(), c->stream, k, sV, vl, sR, M.act.as<int>());
             launch_finalize(is_float, kc, h1, h2, M.Pn.as<double>(), Z, n, basis(kc),
                             M.H.as<double>(), c->stream, k, vl, sV, sR, sH, M.act.as<int>());
             HIPCHK(hipMemcpyAsync(M.hpin, M.H.p, sizeof(double) * sH * k, hipMemcpyDeviceToHost,

@@ -364,16 +364,12 @@ int krylov_partials_blocks(int n);
 void launch_dot_partials(int is_float, const void *V, size_t ldv, int kcount, const void *z,
                          int n, double *P, hipStream_t s, int batch = 1, size_t sV = 0,
                          size_t sZ = 0, const int *active = nullptr);
-// h[b*sH + k] = sum over chunks of the partials P (k < kcount)
-void launch_reduce_parts(int kcount, const double *P, int n, double *h, hipStream_t s,
-                         int batch = 1, size_t sH = 0, const int *active = nullptr);
-// Pin: h is reduced here from the previous pass's chunk partials (h unused), workgroup 0
-// storing it to hsave
-void launch_update_dot(int is_float, const void *V, size_t ldv, int kcount, const double *h,
-                       void *z, int n, double *Pout, double *normp, int want_norm, hipStream_t s,
-                       int batch = 1, size_t sV = 0, size_t sZ = 0, size_t sH = 0,
-                       const int *active = nullptr, const double *Pin = nullptr,
-                       double *hsave = nullptr);
+// z -= V h, h[b*sH + k] the sum over the chunks of the previous pass's partials Pin, stored
+// to hsave; then the partial dots of z (Pout) and partial |z|^2 (normp), either may be null
+void launch_update_dot(int is_float, const void *V, size_t ldv, int kcount, void *z, int n,
+                       const double *Pin, double *hsave, double *Pout, double *normp,
+                       hipStream_t s, int batch = 1, size_t sV = 0, size_t sZ = 0,
+                       size_t sH = 0, const int *active = nullptr);
 // hmap/hseq/seq: also publish hout (kcount + 1 values, single instance) to coherent pinned
 // host memory, then seq to *hseq; xcl/pos (FP32, single instance): also xcl[pos[i]] = vout[i]
 void launch_finalize(int is_float, int kcount, const double *h1, const double *h2,
