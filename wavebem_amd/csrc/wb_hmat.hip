@@ -73,28 +73,32 @@ __device__ __forceinline__ float lane63(float v)
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
-// Wavefront sums of 8 values at once (a transposing reduction): each step pairs a lane
-// with a partner that holds the same set of value indices, keeps half of them and adds
-// the partner's copy of that half (row_mirror splits on lane bit 3, row_half_mirror on
-// bit 2, quad_perm [2,3,0,1] on bit 1); then the lane pairs, the rows and the row pairs
-// are summed.  On return lane l holds the total of value ((l >> 1) & 7): 7 + 3 + 1 DPP
-// adds and 2 cross-row shuffles where 8 separate sums take 8 x 6.
+// Wavefront sums of 8 values at once (a transposing reduction): two lane-swap steps halve
+// the values a lane holds, across the wavefront's halves and then its rows of 16 (a swap
+// and one add for two values); row_mirror splits the last pair on lane bit 3 and the
+// remaining 8 lanes are summed.  On return lane l holds the total of value l / 8: 7 + 3
+// adds in all, none of the steps through LDS.
 __device__ __forceinline__ float wave_sum8(const float (&p)[8])
 {
-    const unsigned l = threadIdx.x & 63u;
-    const bool b3 = l & 8u, b2 = l & 4u, b1 = l & 2u;
     float a[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-        a[j] = (b3 ? p[j + 4] : p[j]) + WB_DPP_MOV(b3 ? p[j] : p[j + 4], 0x140);
+    for (int j = 0; j < 4; ++j) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[j]),
+                                                        __float_as_uint(p[j + 4]), false, false);
+        a[j] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
     float c[2];
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-        c[j] = (b2 ? a[j + 2] : a[j]) + WB_DPP_MOV(b2 ? a[j] : a[j + 2], 0x141);
-    float t = (b1 ? c[1] : c[0]) + WB_DPP_MOV(b1 ? c[0] : c[1], 0x4e);
+    for (int j = 0; j < 2; ++j) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a[j]),
+                                                        __float_as_uint(a[j + 2]), false, false);
+        c[j] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    const bool b3 = threadIdx.x & 8u;
+    float t = (b3 ? c[1] : c[0]) + WB_DPP_MOV(b3 ? c[0] : c[1], 0x140);
+    t += WB_DPP_MOV(t, 0x141);
+    t += WB_DPP_MOV(t, 0x4e);
     t += WB_DPP_MOV(t, 0xb1);
-    t += __shfl_xor(t, 16);
-    t += __shfl_xor(t, 32);
     return t;
 }
 
@@ -721,7 +725,7 @@ __global__ __launch_bounds__(64) void k_hm_gemv_multi(
                     for (int v = 0; v < HM_KV; ++v)
                         if (v < k) {
                             const float t =
-                                __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ts), 2 * v)) *
+                                __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ts), 8 * v)) *
                                 fs;
 #pragma unroll
                             for (int c = 0; c < 4; ++c)
