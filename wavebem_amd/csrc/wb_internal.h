@@ -370,14 +370,14 @@ void launch_update_dot(int is_float, const void *V, size_t ldv, int kcount, void
                        const double *Pin, double *hsave, double *Pout, double *normp,
                        hipStream_t s, int batch = 1, size_t sV = 0, size_t sZ = 0,
                        size_t sH = 0, const int *active = nullptr);
-// hmap/hseq/seq: also publish hout (kcount + 1 values, single instance) to coherent pinned
-// host memory, then seq to *hseq; xcl/pos (FP32, single instance): also xcl[pos[i]] = vout[i]
+// hmap/hseq/seq: also publish hout (kcount + 1 values) to coherent pinned host memory, then
+// seq to *hseq (instance b sHmap entries further on in both); z is only read when vout is; xcl/pos (FP32, single instance): also xcl[pos[i]] = vout[i]
 void launch_finalize(int is_float, int kcount, const double *h1, const double *h2,
                      const double *Pn, void *z, int n, void *vout, double *hout, hipStream_t s,
                      int batch = 1, size_t sZ = 0, size_t sV = 0, size_t sHin = 0,
                      size_t sH = 0, const int *active = nullptr, double *hmap = nullptr,
                      unsigned long long *hseq = nullptr, unsigned long long seq = 0,
-                     float *xcl = nullptr, const int *pos = nullptr);
+                     float *xcl = nullptr, const int *pos = nullptr, size_t sHmap = 0);
 #ifndef WB_ARNOLDI1_KB
 #define WB_ARNOLDI1_KB 160
 #endif
@@ -388,9 +388,9 @@ void launch_arnoldi1(int is_float, const void *V, size_t ldv, int kcount, const 
                      void *vout, double *hout, hipStream_t s, double *hmap,
                      unsigned long long *hseq, unsigned long long seq, float *xcl,
                      const int *pos);
+// x += V y, y (host, kcount entries) taken along as a launch argument
 void launch_axpy_basis(int is_float, const void *V, size_t ldv, int kcount, const double *y,
-                       void *x_acc, int x_is_float, int n, hipStream_t s, int batch = 1,
-                       size_t sV = 0, size_t sY = 0, size_t sX = 0, const int *active = nullptr);
+                       void *x_acc, int x_is_float, int n, hipStream_t s);
 void launch_norm2_partials(int is_float, const void *x, int n, double *P, hipStream_t s,
                            int batch = 1, size_t sX = 0, const int *active = nullptr);
 void launch_vec_ops(int op, int n, const void *a, const void *b, void *c, double alpha,

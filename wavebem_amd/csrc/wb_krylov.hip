@@ -156,15 +156,15 @@ __global__ __launch_bounds__(KTHREADS) void k_update_dot(const T *__restrict__ V
 
 // hout[k] = h1[k] + h2[k] (k < kcount), hout[kcount] = sqrt(sum Pn); vout = z / hout[kcount].
 // Every workgroup forms the norm itself, wavefront-parallel and in the same order.
-// With hmap (coherent pinned host memory, single instance), the column also goes to the
-// host: every thread of workgroup 0 writes its entries and fences at system scope, then
+// With hmap (coherent pinned host memory, instance b at sHmap entries), the column also goes
+// to the host: every thread of workgroup 0 writes its entries and fences at system scope, then
 // thread 0 publishes seq after them, so a host that reads seq (acquire) sees the column.
 // With xcl (single instance), vout is also written to xcl[pos[i]] (FP32).
 template <typename T>
 __global__ __launch_bounds__(KTHREADS) void k_finalize(int kcount, const double *__restrict__ h1,
                                                        const double *__restrict__ h2,
                                                        size_t sHin,
-                                                       const double *__restrict__ Pn,
+                                                       const double *__restrict__ Pn, int nparts,
                                                        const T *__restrict__ z, size_t sZ,
                                                        int n, T *__restrict__ vout, size_t sV,
                                                        double *__restrict__ hout, size_t sH,
@@ -173,18 +173,22 @@ __global__ __launch_bounds__(KTHREADS) void k_finalize(int kcount, const double 
                                                        unsigned long long *__restrict__ hseq,
                                                        unsigned long long seq,
                                                        float *__restrict__ xcl,
-                                                       const int *__restrict__ pos)
+                                                       const int *__restrict__ pos,
+                                                       size_t sHmap)
 {
     __shared__ double snorm;
     const int b = blockIdx.y;
     if (active && !active[b]) return;
-    const int nparts = gridDim.x;
     if (h1) h1 += b * sHin;
     if (h2) h2 += b * sHin;
     Pn += (size_t)b * nparts;
     z += b * sZ;
     if (vout) vout += b * sV;
     hout += b * sH;
+    if (hmap) {
+        hmap += b * sHmap;
+        hseq += b * sHmap;
+    }
     if (threadIdx.x < 64) {
         double s = 0.0;
         for (int p = threadIdx.x; p < nparts; p += 64) s += Pn[p];
@@ -297,23 +301,18 @@ __global__ __launch_bounds__(A1_THREADS) void k_arnoldi1(
 }
 
 // x += sum_i y_i v_i   (x may be double while V is float)
+struct Coefficients {
+    double v[KMAX];
+};
+
 template <typename T, typename TX>
-__global__ void k_axpy_basis(const T *__restrict__ V, size_t ldv, size_t sV, int kcount,
-                             const double *__restrict__ y, size_t sY, TX *__restrict__ x,
-                             size_t sX, int n, const int *__restrict__ active)
+__global__ void k_axpy_basis(const T *__restrict__ V, size_t ldv, int kcount, Coefficients y,
+                             TX *__restrict__ x, int n)
 {
-    __shared__ double ys[KMAX];
-    const int b = blockIdx.y;
-    if (active && !active[b]) return;
-    V += b * sV;
-    y += b * sY;
-    x += b * sX;
-    for (int k = threadIdx.x; k < kcount; k += blockDim.x) ys[k] = y[k];
-    __syncthreads();
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     double a = (double)x[i];
-    for (int k = 0; k < kcount; ++k) a += ys[k] * (double)V[(size_t)k * ldv + i];
+    for (int k = 0; k < kcount; ++k) a += y.v[k] * (double)V[(size_t)k * ldv + i];
     x[i] = (TX)a;
 }
 
@@ -381,17 +380,19 @@ void launch_finalize(int is_float, int kcount, const double *h1, const double *h
                      const double *Pn, void *z, int n, void *vout, double *hout, hipStream_t s,
                      int batch, size_t sZ, size_t sV, size_t sHin, size_t sH,
                      const int *active, double *hmap, unsigned long long *hseq,
-                     unsigned long long seq, float *xcl, const int *pos)
+                     unsigned long long seq, float *xcl, const int *pos, size_t sHmap)
 {
-    dim3 grid(krylov_partials_blocks(n), batch);
+    // without a new vector one workgroup per instance has all there is to do
+    const int parts = krylov_partials_blocks(n);
+    dim3 grid(vout ? parts : 1, batch);
     if (is_float)
         hipLaunchKernelGGL(k_finalize<float>, grid, dim3(KTHREADS), 0, s, kcount, h1, h2, sHin,
-                           Pn, (const float *)z, sZ, n, (float *)vout, sV, hout, sH, active,
-                           hmap, hseq, seq, xcl, pos);
+                           Pn, parts, (const float *)z, sZ, n, (float *)vout, sV, hout, sH,
+                           active, hmap, hseq, seq, xcl, pos, sHmap);
     else
         hipLaunchKernelGGL(k_finalize<double>, grid, dim3(KTHREADS), 0, s, kcount, h1, h2, sHin,
-                           Pn, (const double *)z, sZ, n, (double *)vout, sV, hout, sH, active,
-                           hmap, hseq, seq, (float *)nullptr, pos);
+                           Pn, parts, (const double *)z, sZ, n, (double *)vout, sV, hout, sH,
+                           active, hmap, hseq, seq, (float *)nullptr, pos, sHmap);
 }
 
 // Whether an Arnoldi step with kcount basis vectors goes to k_arnoldi1: the basis it reads
@@ -419,19 +420,20 @@ void launch_arnoldi1(int is_float, const void *V, size_t ldv, int kcount, const 
 }
 
 void launch_axpy_basis(int is_float, const void *V, size_t ldv, int kcount, const double *y,
-                       void *x, int x_is_float, int n, hipStream_t s, int batch, size_t sV,
-                       size_t sY, size_t sX, const int *active)
+                       void *x, int x_is_float, int n, hipStream_t s)
 {
-    dim3 grid((n + 255) / 256, batch);
+    Coefficients yv;
+    for (int k = 0; k < kcount; ++k) yv.v[k] = y[k];
+    const dim3 grid((n + 255) / 256);
     if (is_float && x_is_float)
         hipLaunchKernelGGL((k_axpy_basis<float, float>), grid, dim3(256), 0, s, (const float *)V,
-                           ldv, sV, kcount, y, sY, (float *)x, sX, n, active);
+                           ldv, kcount, yv, (float *)x, n);
     else if (is_float)
         hipLaunchKernelGGL((k_axpy_basis<float, double>), grid, dim3(256), 0, s,
-                           (const float *)V, ldv, sV, kcount, y, sY, (double *)x, sX, n, active);
+                           (const float *)V, ldv, kcount, yv, (double *)x, n);
     else
         hipLaunchKernelGGL((k_axpy_basis<double, double>), grid, dim3(256), 0, s,
-                           (const double *)V, ldv, sV, kcount, y, sY, (double *)x, sX, n, active);
+                           (const double *)V, ldv, kcount, yv, (double *)x, n);
 }
 
 void launch_norm2_partials(int is_float, const void *x, int n, double *P, hipStream_t s,
