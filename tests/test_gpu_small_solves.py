@@ -55,3 +55,32 @@ def test_small_arnoldi_limits(n):
     b, sb = _solve(m, bc, precision="fp32_ir")
     assert sa["true_rel_residual"] < 1e-9 and sb["true_rel_residual"] < 1e-9
     assert np.abs(a - b).max() < 1e-8 * np.abs(a).max()
+
+
+# constraint lines written by the product's launch: none, and 52 and 112 of them (less than a
+# wavefront, a part of a block)
+@pytest.mark.parametrize("n, lines", [(4, False), (4, True), (9, True)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32_ir"])
+def test_product_writes_constraint_lines(n, lines, precision):
+    m = M.box_mesh(n=n, hi=(1.0, 0.8, 0.6), dirichlet_top=True)
+    ptr, idx = M.double_nodes_csr(m.support_points)
+    H, G = O.assemble(m.support_points, m.cell_dofs, m.cell_orient, ptr, idx)
+    rng = np.random.default_rng(n)
+    bc = rng.standard_normal(m.n_dofs)[[idx[a] for a in ptr[:-1]]]
+    src = rng.standard_normal(m.n_dofs)
+    with BEMProblem(m, Config(precision=precision)) as p:
+        if lines:
+            p.compute_constraints(bc)
+        else:
+            p.set_constraints([], [0], [], [], [])
+        p.assemble_system()
+        dst = p.constrained_vmult(src)
+    if lines:
+        cons = O.compute_constraints(ptr, idx, m.surface_nodes, bc)
+        A, _ = T.explicit_system(H, G, m.surface_nodes, m.other_nodes, cons, bc)
+        want = A @ src
+    else:
+        want = O.vmult(G, H, O.compute_alpha(H), m.surface_nodes, m.other_nodes, src)
+    # FP64: sums of n products; FP32-IR: entries to 2^-33
+    tol = 1e-12 if precision == "fp64" else 1e-9
+    assert np.abs(dst - want).max() < tol * np.abs(want).max()

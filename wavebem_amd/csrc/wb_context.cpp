@@ -486,8 +486,15 @@ static void hm_product(wb_ctx *c, const void *x, void *y, bool lines, bool cpart
                    cparts ? c->cs_agg : 64, cparts ? c->cs_Cpart.as<double>() : nullptr);
 }
 
+static ConLines con_lines(const wb_ctx *c)
+{
+    return {c->n_lines, c->con_rows.as<int>(), c->con_ptr.as<int>(), c->con_cols.as<int>(),
+            c->con_w.as<double>()};
+}
+
+// with lines (modes 0 to 2), constrained rows get their line's value in the same launch
 static void gemv(wb_ctx *c, int mode, int which, const void *x, const void *xd, void *y,
-                 bool free_rows_only)
+                 bool free_rows_only, bool lines = false)
 {
     const double *diag = which == 0 ? c->diag_op.as<double>() : c->diag_rhs.as<double>();
     const double s_sel = which == 0 ? 1.0 : -1.0, s_uns = which == 0 ? -1.0 : 1.0;
@@ -509,7 +516,7 @@ static void gemv(wb_ctx *c, int mode, int which, const void *x, const void *xd, 
     KernelScope ks(c, mode == 0 ? WB_K_GEMV64 : (mode == 1 ? WB_K_GEMV32 : WB_K_GEMVHL), nr);
     launch_gemv_sel(mode, c->G.p, c->H.p, c->Glo.p, c->Hlo.p, c->ld, c->segs.as<int>(),
                     c->n_segs, c->gmask.as<uint8_t>(), which, s_sel, s_uns, x, diag, xd, rows, nr,
-                    y, c->stream);
+                    y, c->stream, lines ? con_lines(c) : ConLines{});
 }
 
 // y = ConstrainedOperator(A) x in FP64 (mode 0 or 2) or FP32 vectors (mode 1: FP32
@@ -569,7 +576,8 @@ static bool apply_constrained(wb_ctx *c, int mode, const void *x, void *y,
             HIPCHK(hipMemcpy(y, v.data(), sizeof(double) * c->n, hipMemcpyHostToDevice));
         }
     } else {
-        gemv(c, mode, 0, x, x, y, true);
+        gemv(c, mode, 0, x, x, y, true, mode <= 2);
+        if (mode <= 2) return false;
     }
     launch_constraint_rows(is_float, c->n_lines, c->con_rows.as<int>(), c->con_ptr.as<int>(),
                            c->con_cols.as<int>(), c->con_w.as<double>(),
@@ -2507,10 +2515,8 @@ wb_status wb_constrained_vmult_noalloc(wb_ctx *c, const double *src, double *dst
         const int mode = c->cfg.precision == WB_PREC_FP64 ? 0 : 2;
         launch_gemv_sel(mode, c->G.p, c->H.p, c->Glo.p, c->Hlo.p, c->ld, c->segs.as<int>(),
                         c->n_segs, c->gmask.as<uint8_t>(), 0, 1.0, -1.0, xs,
-                        c->diag_op.as<double>(), xs, c->free_rows.as<int>(), c->n_free, ys, s);
-        launch_constraint_rows(0, c->n_lines, c->con_rows.as<int>(), c->con_ptr.as<int>(),
-                               c->con_cols.as<int>(), c->con_w.as<double>(),
-                               c->con_inhom.as<double>(), 0, xs, ys, s);
+                        c->diag_op.as<double>(), xs, c->free_rows.as<int>(), c->n_free, ys, s,
+                        con_lines(c));
         launch_permute(c->n, c->perm_d.as<int>(), ys, dst, 1, s);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(s));

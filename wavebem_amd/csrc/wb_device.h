@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "wb_internal.h"
+
 namespace wb {
 
 // 1/sqrt(r2) in FP64 from the hardware estimate y0 (relative error eps).
@@ -141,6 +143,15 @@ __device__ int gj_invert_lds(T *A, T *colk, int *piv, int *red_i, int bs)
         __syncthreads();
     }
     return zero_pivots;
+}
+
+// value of constraint line l for the vector x
+template <typename T>
+__device__ __forceinline__ double line_value(const ConLines &L, int l, const T *__restrict__ x)
+{
+    double v = (double)x[L.rows[l]];
+    for (int p = L.ptr[l]; p < L.ptr[l + 1]; ++p) v -= L.w[p] * (double)x[L.cols[p]];
+    return v;
 }
 
 }  // namespace wb

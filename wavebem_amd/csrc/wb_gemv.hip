@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "wb_internal.h"
+#include "wb_device.h"
 
 namespace wb {
 
@@ -53,15 +54,30 @@ __device__ __forceinline__ void load_rows(int slot0, const int *__restrict__ row
 
 constexpr int F64_RPW = 4, F64_WAVES = 4;
 
+// The blocks past those of the n_rows rows (PB each) write the constraint lines, one thread
+// per line; returns whether this is one of them.  (A launch of its own took 4 us and the gap
+// before it: an FP64 step at 2.9k dofs 2.18 -> 2.12 ms, one product at 1,083 dofs 57 -> 54 us.)
+template <int PB, typename T>
+__device__ __forceinline__ bool lines_block(int n_rows, const ConLines &L,
+                                            const T *__restrict__ x, T *__restrict__ y)
+{
+    const int b = (int)blockIdx.x - (n_rows + PB - 1) / PB;
+    if (b < 0) return false;
+    const int l = b * (int)blockDim.x + (int)threadIdx.x;
+    if (l < L.n) y[L.rows[l]] = (T)line_value(L, l, x);
+    return true;
+}
+
 // segment = int4 {first group, end group, kind (0 G, 1 H, 2 mixed), unused}
 __global__ __launch_bounds__(64 * F64_WAVES) void k_gemv_f64(
     const double *__restrict__ G, const double *__restrict__ H, size_t ld,
     const int4 *__restrict__ segs, int n_segs, const uint8_t *__restrict__ gmask, int flip,
     double s_sel, double s_uns, const double *__restrict__ x, const double *__restrict__ diag,
     const double *__restrict__ xd, const int *__restrict__ rows, int n_rows,
-    double *__restrict__ y)
+    double *__restrict__ y, ConLines lines)
 {
     constexpr int RPW = F64_RPW;
+    if (lines_block<F64_RPW * F64_WAVES>(n_rows, lines, x, y)) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int r[RPW];
     bool ok[RPW];
@@ -131,6 +147,7 @@ template <int MODE> struct MixedShape;
 #define WB_GEMV32_RPW 4
 #endif
 template <> struct MixedShape<1> {
+    typedef float V;
     static constexpr int RPW = WB_GEMV32_RPW, WAVES = 16 / WB_GEMV32_RPW;
 };
 #ifndef WB_GEMVHL_RPW
@@ -143,6 +160,7 @@ template <> struct MixedShape<1> {
 #define WB_GEMVHL_UNROLL 2
 #endif
 template <> struct MixedShape<2> {
+    typedef double V;
     static constexpr int RPW = WB_GEMVHL_RPW, WAVES = WB_GEMVHL_WAVES;
 };
 
@@ -152,9 +170,11 @@ __global__ __launch_bounds__(64 * MixedShape<MODE>::WAVES) void k_gemv_mixed(
     const uint16_t *__restrict__ Hlo, size_t ld, const int4 *__restrict__ segs, int n_segs,
     const uint8_t *__restrict__ gmask, int flip, double s_sel, double s_uns,
     const void *__restrict__ xv_, const double *__restrict__ diag, const void *__restrict__ xd_,
-    const int *__restrict__ rows, int n_rows, void *__restrict__ y_)
+    const int *__restrict__ rows, int n_rows, void *__restrict__ y_, ConLines lines)
 {
     constexpr int RPW = MixedShape<MODE>::RPW, WAVES = MixedShape<MODE>::WAVES;
+    typedef typename MixedShape<MODE>::V V;
+    if (lines_block<RPW * WAVES>(n_rows, lines, (const V *)xv_, (V *)y_)) return;
     typedef double T;  // products and sums in FP64 in both modes
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int r[RPW];
@@ -551,32 +571,30 @@ void launch_gemv_h16(const void *A16, const float *rs, size_t ld, int n, const f
 void launch_gemv_sel(int mode, const void *G, const void *H, const void *Glo, const void *Hlo,
                      size_t ld, const int *segs, int n_segs, const uint8_t *gmask, int flip,
                      double s_sel, double s_unsel, const void *x, const double *diag,
-                     const void *xd, const int *rows, int n_rows, void *y, hipStream_t s)
+                     const void *xd, const int *rows, int n_rows, void *y, hipStream_t s,
+                     const ConLines &lines)
 {
-    if (n_rows <= 0) return;
+    n_rows = n_rows < 0 ? 0 : n_rows;
+    if (n_rows == 0 && lines.n <= 0) return;
+    auto grid = [&](int per_block, int threads) {
+        return dim3((n_rows + per_block - 1) / per_block + (lines.n + threads - 1) / threads);
+    };
     if (mode == 0) {
-        const int per_block = F64_RPW * F64_WAVES;
-        hipLaunchKernelGGL(k_gemv_f64, dim3((n_rows + per_block - 1) / per_block),
+        hipLaunchKernelGGL(k_gemv_f64, grid(F64_RPW * F64_WAVES, 64 * F64_WAVES),
                            dim3(64 * F64_WAVES), 0, s, (const double *)G, (const double *)H, ld,
                            (const int4 *)segs, n_segs, gmask, flip, s_sel, s_unsel,
-                           (const double *)x, diag, (const double *)xd, rows, n_rows, (double *)y);
+                           (const double *)x, diag, (const double *)xd, rows, n_rows, (double *)y,
+                           lines);
         return;
     }
-    if (mode == 1) {
-        constexpr int pb = MixedShape<1>::RPW * MixedShape<1>::WAVES;
-        hipLaunchKernelGGL(k_gemv_mixed<1>, dim3((n_rows + pb - 1) / pb),
-                           dim3(64 * MixedShape<1>::WAVES), 0, s, (const float *)G,
-                           (const float *)H, (const uint16_t *)Glo, (const uint16_t *)Hlo, ld,
-                           (const int4 *)segs, n_segs, gmask, flip, s_sel, s_unsel, x, diag, xd,
-                           rows, n_rows, y);
-    } else {
-        constexpr int pb = MixedShape<2>::RPW * MixedShape<2>::WAVES;
-        hipLaunchKernelGGL(k_gemv_mixed<2>, dim3((n_rows + pb - 1) / pb),
-                           dim3(64 * MixedShape<2>::WAVES), 0, s, (const float *)G,
-                           (const float *)H, (const uint16_t *)Glo, (const uint16_t *)Hlo, ld,
-                           (const int4 *)segs, n_segs, gmask, flip, s_sel, s_unsel, x, diag, xd,
-                           rows, n_rows, y);
-    }
+    auto mixed = [&](auto kern, int rpw, int waves) {
+        hipLaunchKernelGGL(kern, grid(rpw * waves, 64 * waves), dim3(64 * waves), 0, s,
+                           (const float *)G, (const float *)H, (const uint16_t *)Glo,
+                           (const uint16_t *)Hlo, ld, (const int4 *)segs, n_segs, gmask, flip,
+                           s_sel, s_unsel, x, diag, xd, rows, n_rows, y, lines);
+    };
+    if (mode == 1) mixed(k_gemv_mixed<1>, MixedShape<1>::RPW, MixedShape<1>::WAVES);
+    else mixed(k_gemv_mixed<2>, MixedShape<2>::RPW, MixedShape<2>::WAVES);
 }
 
 }  // namespace wb

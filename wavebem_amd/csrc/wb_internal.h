@@ -239,10 +239,19 @@ void launch_alpha_reduce(const double *hsum_part, int n_parts, const double *hsu
 // sel bit per column pair in pairflag (0: G,G 1: H,H 2: G,H 3: H,G), flipped by `flip`.
 // mode: 0 = FP64 matrices, 1 = hi only (FP32 accumulate), 2 = hi+lo (FP64 accumulate)
 // segs: n_segs x int4 {first 4-column group, end group, kind 0=G 1=H 2=mixed, 0}
+// Constraint lines of a product (n = 0: none): y[rows[l]] = x[rows[l]] - sum_p w[p] x[cols[p]],
+// p from ptr[l] to ptr[l + 1]
+struct ConLines {
+    int n = 0;
+    const int *rows = nullptr, *ptr = nullptr, *cols = nullptr;
+    const double *w = nullptr;
+};
+// (lines: written by the same launch; their rows are not among rows)
 void launch_gemv_sel(int mode, const void *G, const void *H, const void *Glo, const void *Hlo,
                      size_t ld, const int *segs, int n_segs, const uint8_t *gmask, int flip,
                      double s_sel, double s_unsel, const void *x, const double *diag,
-                     const void *xd, const int *rows, int n_rows, void *y, hipStream_t s);
+                     const void *xd, const int *rows, int n_rows, void *y, hipStream_t s,
+                     const ConLines &lines = ConLines{});
 // k <= 16 vectors at once (column v at X + v*ldx, Xd + v*ldx, Y + v*ldy) on the matrix
 // cores; the columns are split into multi_chunks(mode, n_rows, n_groups) chunks whose
 // partials (part: chunks * k * n_rows doubles) are added in order.  Mode 3 (FP16 operator)

@@ -8,7 +8,7 @@
 // agree (all but the few at a Dirichlet/Neumann boundary in the device ordering) issue
 // one vector load from the selected matrix.  Rows run one per (wave, row slot) with
 // wavefront shuffle reductions; constrained rows (ConstrainedOperator,
-// include/constrained_matrix.h:73-86) are skipped and rewritten by a small fix-up kernel.
+// include/constrained_matrix.h:73-86) are skipped; blocks of the same launch write their lines.
 #include "wb_internal.h"
 #include "wb_device.h"
 
@@ -52,9 +52,7 @@ __global__ void k_constraint_rows(int n_lines, const int *__restrict__ rows,
         y[r] = (T)inhom[l];
         return;
     }
-    double v = (double)x[r];
-    for (int p = ptr[l]; p < ptr[l + 1]; ++p) v -= w[p] * (double)x[cols[p]];
-    y[r] = (T)v;
+    y[r] = (T)line_value({n_lines, rows, ptr, cols, w}, l, x);
 }
 
 // op[i] = alpha[i] (1 - s[i]), rhs[i] = -alpha[i] s[i] for a 0/1 mask s
