@@ -747,12 +747,19 @@ __global__ __launch_bounds__(256) void k_assemble_singular(
         for (int o = SING_LANES / 2; o > 0; o >>= 1)
 #pragma unroll
             for (int k = 0; k < 8; ++k) lv[k] += __shfl_xor(lv[k], o, 64);
-        // every lane holds the sums: lane k < 4 adds entry k of G, lane 4 + k of H
+        // every lane holds the sums: lane k < 4 adds entry vid[k] of G, lane 4 + k of H; of
+        // lanes with the same entry (a cell that names a dof twice) the first adds their sum
+        const int vk = sl & 2 ? (sl & 1 ? vid[3] : vid[2]) : (sl & 1 ? vid[1] : vid[0]);
         double add = 0.0;
+        bool first = sl < 8;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) add = sl == k ? lv[k] : add;
-        if (sl < 8) {
-            const size_t off = (size_t)i * ld + vid[sl & 3];
+        for (int j = 0; j < 4; ++j) {
+            const bool same = vid[j] == vk;
+            add += same ? (sl < 4 ? lv[j] : lv[4 + j]) : 0.0;
+            first = first && !(same && j < (sl & 3));
+        }
+        if (first) {
+            const size_t off = (size_t)i * ld + vk;
             void *M = sl < 4 ? Gv : Hv;
             add *= sl < 4 ? INV4PI : -INV4PI;
             if (OUT == 0) {
