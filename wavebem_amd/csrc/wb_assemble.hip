@@ -774,6 +774,10 @@ __global__ __launch_bounds__(256) void k_assemble_singular(
             }
         }
         for (int k = 0; k < 4; ++k) hs += lv[4 + k] * (-INV4PI);
+        // the next cell shares vertices with this one under other k: what a lane has stored is
+        // another lane's load there (one wavefront: program order of its memory operations)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
     if (sl == 0) hsum_sing[i] = hs;
 }
