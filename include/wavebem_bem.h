@@ -421,6 +421,10 @@ int wb_host_cluster_plan(int n_dofs, int n_cells, const double *support_points,
 int wb_host_hm_work_items(int n_clusters, const uint8_t *rank, const int32_t *cl_size,
                           int32_t *sizes, int32_t *item_ptr, int32_t *items);
 
+/* Device memory that wb_residual_vjp takes besides vectors, for n_dofs rows and n_cells
+ * cells: bytes[0..2] = point records, partial sums by row, partial sums by point. */
+int wb_host_adjoint_scratch(int n_dofs, int n_cells, int q_order, int64_t *bytes);
+
 /* BEMProblem::compute_constraints (source/bem_problem.cc:990-1105) rules, closed as by
  * ConstraintMatrix::close; returns the number of lines, or minus a wb_status. */
 int wb_host_compute_constraints(int n, const int32_t *dn_ptr, const int32_t *dn_idx,

@@ -76,3 +76,23 @@ def test_device_calls_fail_cleanly_without_gpu():
     assert st in (L.WB_E_HIP, L.WB_OK)
     if st == L.WB_OK:
         L.lib().wb_destroy(ctx)
+
+
+@pytest.mark.parametrize("q", [1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("n", [54, 1083, 10951, 41207, 65536, 65537, 100000, 130000, 155000,
+                               1000000])
+def test_adjoint_scratch_is_bounded(n, q):
+    """The backward's scratch memory: near the largest problems, whose matrices fill the card,
+    linear in the mesh (16 partials of 7 doubles and 2 doubles per point, 64 of 3 per row);
+    below 32k cells enough chunks for 2048 workgroups, which is a constant."""
+    nc = n - n // 50  # closed surfaces have a little fewer cells than dofs
+    b = (ctypes.c_int64 * 3)()
+    assert L.lib().wb_host_adjoint_scratch(n, nc, q, b) == L.WB_OK
+    per_point = (16 * 7 + 2) * 8 * nc * q * q
+    per_row = 64 * 3 * 8 * n
+    pad = 64 * 8
+    if n > 65536:
+        assert b[0] + b[2] <= per_point + pad and b[1] <= per_row
+    # the chunks of 2048 workgroups of 256 points or rows
+    assert b[0] + b[2] <= max(per_point, 72 * nc * q * q + 7 * 8 * 256 * 2048 * 2) + pad
+    assert b[1] <= max(per_row, 3 * 8 * 256 * 2048 * 2)

@@ -818,23 +818,32 @@ void launch_constraint_T(int is_float, int n_targets, const int *tgt, const int 
 }
 
 // Chunks of the cells for the row passes: at least 2048 workgroups of 256 rows (a CU holds
-// four), at most 1024 cells and at least 16 in a chunk.
+// four), at most 1024 cells and at least 16 in a chunk; at most 64 chunks beyond what 2048
+// workgroups take, since every chunk is a partial per row.
 int vjp_row_chunks(int n, int nc)
 {
     const int blocks = (n + 255) / 256;
-    const int want = max((nc + 1023) / 1024, (2048 + blocks - 1) / blocks);
+    const int want = max(min(64, (nc + 1023) / 1024), (2048 + blocks - 1) / blocks);
     return max(1, min(want, (nc + 15) / 16));
 }
 // Chunks of the rows for the point pass, likewise: at least 2048 workgroups of four
-// wavefronts, at least 128 rows in a chunk.
+// wavefronts, at least 128 rows in a chunk, at most 15 chunks beyond that: a chunk is 56
+// bytes per point, and the matrices of the largest problems fill the card (15 chunks and the
+// point records of 72 bytes are 1.9 GB at 130k rows and the 4x4 rule).
 int vjp_point_chunks(int n, int nc, int nq)
 {
     const int blocks = (nc + 4 * (64 / nq) - 1) / (4 * (64 / nq));
-    const int want = max((n + 4095) / 4096, (2048 + blocks - 1) / blocks);
+    const int want = max(min(15, (n + 4095) / 4096), (2048 + blocks - 1) / blocks);
     return max(1, min(want, (n + 127) / 128));
 }
 // doubles of the point records (with padding) and of Psi after them
 size_t adj_record_doubles(int nc, int nq) { return 8 * ((size_t)nc * nq + REC_PAD); }
+
+VjpScratch vjp_scratch(int n, int nc, int nq)
+{
+    return {adj_record_doubles(nc, nq) + (size_t)nc * nq, (size_t)vjp_row_chunks(n, nc) * n * 3,
+            (size_t)vjp_point_chunks(n, nc, nq) * nc * nq * 7};
+}
 
 void launch_residual_vjp(int q_order, int n, int nc, const double *X, const int *row_cls,
                          const double *wrow, const double *phi, const double *psi,

@@ -2701,10 +2701,10 @@ wb_status wb_residual_vjp(wb_ctx *c, const double *w, const double *phi, const d
         upload(c->vjp_psi, si.data(), n, c->stream);
         upload(c->vjp_rows, rp.data(), rp.size(), c->stream);
         const int npairs = (int)c->plan.sing_cell.size();
-        // point records and Psi
-        c->vjp_cstate.ensure(sizeof(double) * (adj_record_doubles(nc, nq) + (size_t)nc * nq));
-        c->vjp_p1.ensure(sizeof(double) * 3 * (size_t)vjp_row_chunks(n, nc) * n);
-        c->vjp_p2.ensure(sizeof(double) * 7 * (size_t)vjp_point_chunks(n, nc, nq) * nc * nq);
+        const VjpScratch vs = vjp_scratch(n, nc, nq);
+        c->vjp_cstate.ensure(sizeof(double) * vs.cstate);
+        c->vjp_p1.ensure(sizeof(double) * vs.part1);
+        c->vjp_p2.ensure(sizeof(double) * vs.part2);
         c->vjp_xg.ensure(sizeof(double) * 3 * (size_t)n);
         c->vjp_vbar.ensure(sizeof(double) * 12 * (size_t)nc);
         c->vjp_xs.ensure(sizeof(double) * 3 * (size_t)n);

@@ -110,6 +110,16 @@ int wb_host_hm_work_items(int ncl, const uint8_t *rank, const int32_t *cl_size,
     return WB_OK;
 }
 
+int wb_host_adjoint_scratch(int n, int nc, int q_order, int64_t *bytes)
+{
+    if (n <= 0 || nc <= 0 || q_order < 1 || q_order > wb::MAX_NQ1 || !bytes) return WB_E_ARG;
+    const wb::VjpScratch s = wb::vjp_scratch(n, nc, q_order * q_order);
+    bytes[0] = (int64_t)(sizeof(double) * s.cstate);
+    bytes[1] = (int64_t)(sizeof(double) * s.part1);
+    bytes[2] = (int64_t)(sizeof(double) * s.part2);
+    return WB_OK;
+}
+
 int wb_host_compute_constraints(int n, const int32_t *dn_ptr, const int32_t *dn_idx,
                                 const double *surface, const double *normals,
                                 const double *grads, const double *tmp_rhs, int cap_lines,

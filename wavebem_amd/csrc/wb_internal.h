@@ -350,12 +350,14 @@ void launch_gemvT(int mode, const void *G, const void *H, const void *Glo, const
 void launch_constraint_T(int is_float, int n_targets, const int *tgt, const int *ptr,
                          const int *src, const double *coef, const void *x, void *y,
                          hipStream_t s);
-// backward of the assembly; buffer sizes: cstate adj_record_doubles + nc*nq,
-// part1 vjp_row_chunks*n*3,
-// part2 vjp_point_chunks*nc*nq*7, rowpack 8*(n + REC_PAD), xgrad n*3, vbar nc*12, xs n*3, spart n_sing*12
+// backward of the assembly; buffer sizes: cstate, part1 and part2 as vjp_scratch, rowpack
+// 8*(n + REC_PAD), xgrad n*3, vbar nc*12, xs n*3, spart n_sing*12
 int vjp_row_chunks(int n, int nc);
-int vjp_point_chunks(int n, int nc, int nq);
 size_t adj_record_doubles(int nc, int nq);
+struct VjpScratch {  // doubles
+    size_t cstate, part1, part2;
+};
+VjpScratch vjp_scratch(int n, int nc, int nq);
 void launch_residual_vjp(int q_order, int n, int nc, const double *X, const int *row_cls,
                          const double *wrow, const double *phi, const double *psi,
                          const double *rowpack, const double *cellq, const int *cell_int,
