@@ -148,11 +148,12 @@ struct wb_ctx {
     int float_mode = 1;  // operator mode of the FP32-vector solves: 1 = FP32 hi, 3 = FP16,
                          // 4 = compressed
     // device: solver work
-    DevBuf V, z, w, P1, P2, Pn, hbuf, hred, vx, vb, vr, vt, vs;   // double / raw
+    DevBuf V, z, w, P1, P2, Pn, hred, vx, vb, vr, vt, vs;   // double / raw
     DevBuf V32, z32, w32, r32, d32;
-    // coherent pinned host memory the GMRES columns are published to: two slots of
-    // HMAP_STRIDE doubles (up to KMAX + 1 values, the sequence number in the last word),
-    // publication seq using slot seq & 1; device-side address of the same memory
+    // coherent pinned host memory that GMRES columns and norms are published to: HMAP_SLOTS
+    // slots of HMAP_STRIDE doubles (up to KMAX + 1 values, the sequence number in the last
+    // word), column hmap_seq in slot hmap_seq & 1, norm norm_seq in NORM_SLOT; device-side
+    // address of the same memory
     double *hmap = nullptr, *hmap_dev = nullptr;
     unsigned long long hmap_seq = 0, norm_seq = 0;
     size_t vlen = 0;         // padded vector length
@@ -173,14 +174,14 @@ struct wb_ctx {
     // several right-hand sides at once
     struct Multi {
         int k = 0;
-        DevBuf V, V32, Z, W, Z32, W32, P1, P2, Pn, H, hred, X, B, R, T, D32, R32, act, inh, part,
+        DevBuf V, V32, Z, W, Z32, W32, P1, P2, Pn, hred, X, B, R, T, D32, R32, act, inh, part,
             xs, hxc, hpart;
         double *hmap = nullptr, *hmap_dev = nullptr;  // 2 x k slots of a GMRES column (as wb_ctx)
         unsigned long long seq = 0;
         int *apin = nullptr;     // pinned k active flags
         std::vector<DevBuf *> all()
         {
-            return {&V, &V32, &Z, &W, &Z32, &W32, &P1, &P2, &Pn, &H, &hred,
+            return {&V, &V32, &Z, &W, &Z32, &W32, &P1, &P2, &Pn, &hred,
                     &X, &B, &R, &T, &D32, &R32, &act, &inh, &part, &xs, &hxc, &hpart};
         }
     } mw;
@@ -197,7 +198,7 @@ struct wb_ctx {
             &con_line, &cs_Cpart, &surf_c,
             &free_rows, &binv, &binv32, &cs_AP, &cs_Ac, &cs_Aci, &cs_Aci32, &cs_WT,
             &cs_WT32, &cs_status, &cs_C, &cs_T, &cs_PTA, &cs_WTT, &cs_S, &V, &z, &w, &P1, &P2,
-            &Pn, &hbuf, &hred, &vx, &vb, &vr, &vt, &vs, &V32, &z32, &w32, &r32, &d32, &ct_tgt,
+            &Pn, &hred, &vx, &vb, &vr, &vt, &vs, &V32, &z32, &w32, &r32, &d32, &ct_tgt,
             &ct_ptr, &ct_src, &ct_coef, &gt_part, &vjp_w, &vjp_phi, &vjp_psi, &vjp_rows,
             &vjp_cstate, &vjp_p1, &vjp_p2, &vjp_xg, &vjp_vbar, &vjp_xs, &vjp_spart, &inc_ptr,
             &inc_item, &pj_emass, &pj_erhs, &pj_u, &pj_psi, &pj_B, &pj_X, &pj_R, &pj_Z, &pj_P,
@@ -394,7 +395,6 @@ static void ensure_work(wb_ctx *c)
     c->P1.ensure(sizeof(double) * parts * 128);
     c->P2.ensure(sizeof(double) * parts * 128);
     c->Pn.ensure(sizeof(double) * parts);
-    c->hbuf.ensure(sizeof(double) * 132);
     c->hred.ensure(sizeof(double) * 2 * KMAX);
     if (!c->hmap) {
         alloc_slots(HMAP_SLOTS, &c->hmap, &c->hmap_dev);
@@ -418,9 +418,8 @@ static void finalize_publish(wb_ctx *c, int is_float, int kcount, const double *
     double *slot = c->hmap_dev + (seq & 1) * HMAP_STRIDE;
     const bool xc = cluster_copy(c, is_float);
     launch_finalize(is_float, kcount, h1, h2, c->Pn.as<double>(), z, n, vout,
-                    c->hbuf.as<double>(), c->stream, 1, 0, 0, 0, 0, nullptr, slot,
-                    (unsigned long long *)(slot + HMAP_STRIDE - 1), seq,
-                    xc ? c->hm_T.as<float>() : nullptr, xc ? c->hm_pos.as<int>() : nullptr);
+                    slot, (unsigned long long *)(slot + HMAP_STRIDE - 1), seq, c->stream, 1, 0,
+                    0, 0, 0, nullptr, xc ? c->hm_T.as<float>() : nullptr, xc ? c->hm_pos.as<int>() : nullptr);
     c->hm_xc_for = xc ? vout : nullptr;
 }
 
@@ -437,7 +436,7 @@ static const double *wait_slot(wb_ctx *c, const double *slot, unsigned long long
             if (e != hipSuccess && e != hipErrorNotReady) HIPCHK(e);
             if (e == hipSuccess) {
                 if (__atomic_load_n(p, __ATOMIC_ACQUIRE) >= seq) return slot;
-                throw WbError(WB_E_HIP, "GMRES column was not published");
+                throw WbError(WB_E_HIP, "a published column or norm did not arrive");
             }
         }
     }
@@ -453,15 +452,13 @@ static const double *wait_hmap(wb_ctx *c, unsigned long long seq)
 // sums to pageable memory and a wait for the stream, together with the coefficients of
 // launch_axpy_basis as a launch argument: 2.03 -> 1.91 ms for a whole FP32-IR step at 1,083
 // unknowns, six norms and four cycles.)
-
 static double device_norm(wb_ctx *c, const void *x, int is_float)
 {
     launch_norm2_partials(is_float, x, c->n, c->Pn.as<double>(), c->stream);
     double *slot = c->hmap_dev + NORM_SLOT * HMAP_STRIDE;
     const unsigned long long sq = ++c->norm_seq;
     launch_finalize(is_float, 0, nullptr, nullptr, c->Pn.as<double>(), nullptr, c->n, nullptr,
-                    c->hbuf.as<double>(), c->stream, 1, 0, 0, 0, 0, nullptr, slot,
-                    (unsigned long long *)(slot + HMAP_STRIDE - 1), sq);
+                    slot, (unsigned long long *)(slot + HMAP_STRIDE - 1), sq, c->stream);
     return wait_slot(c, c->hmap + NORM_SLOT * HMAP_STRIDE, sq)[0];
 }
 
@@ -881,9 +878,8 @@ static GmresResult gmres(wb_ctx *c, int is_float, const void *b, void *x, double
                 const unsigned long long sq = ++c->hmap_seq;
                 double *slot = c->hmap_dev + (sq & 1) * HMAP_STRIDE;
                 const bool xc = cluster_copy(c, is_float);
-                launch_arnoldi1(is_float, V.p, ldv, k + 1, z, n, vec(k + 1),
-                                c->hbuf.as<double>(), c->stream, slot,
-                                (unsigned long long *)(slot + HMAP_STRIDE - 1), sq,
+                launch_arnoldi1(is_float, V.p, ldv, k + 1, z, n, vec(k + 1), slot,
+                                (unsigned long long *)(slot + HMAP_STRIDE - 1), sq, c->stream,
                                 xc ? c->hm_T.as<float>() : nullptr,
                                 xc ? c->hm_pos.as<int>() : nullptr);
                 c->hm_xc_for = xc ? vec(k + 1) : nullptr;
@@ -1397,10 +1393,9 @@ static unsigned long long publish_multi(wb_ctx *c, int is_float, int kcount, con
     auto &M = c->mw;
     const unsigned long long sq = ++M.seq;
     double *slot = M.hmap_dev + (sq & 1) * M.k * HMAP_STRIDE;
-    launch_finalize(is_float, kcount, h1, h2, M.Pn.as<double>(), z, c->n, vout, M.H.as<double>(),
-                    c->stream, k, c->vlen, sV, 2 * KMAX, 132, active, slot,
-                    (unsigned long long *)(slot + HMAP_STRIDE - 1), sq, nullptr, nullptr,
-                    HMAP_STRIDE);
+    launch_finalize(is_float, kcount, h1, h2, M.Pn.as<double>(), z, c->n, vout, slot,
+                    (unsigned long long *)(slot + HMAP_STRIDE - 1), sq, c->stream, k, c->vlen, sV,
+                    2 * KMAX, HMAP_STRIDE, active);
     return sq;
 }
 
@@ -1579,7 +1574,6 @@ static void solve_multi(wb_ctx *c, int k, const double *tmp_rhs, double *phi, do
     M.P1.ensure(sizeof(double) * parts * KMAX * k);
     M.P2.ensure(sizeof(double) * parts * KMAX * k);
     M.Pn.ensure(sizeof(double) * parts * k);
-    M.H.ensure(sizeof(double) * 132 * k);
     M.hred.ensure(sizeof(double) * 2 * KMAX * k);
     M.act.ensure(sizeof(int) * k);
     if (M.k < k) {

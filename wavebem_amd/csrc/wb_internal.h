@@ -381,14 +381,15 @@ void launch_update_dot(int is_float, const void *V, size_t ldv, int kcount, void
                        const double *Pin, double *hsave, double *Pout, double *normp,
                        hipStream_t s, int batch = 1, size_t sV = 0, size_t sZ = 0,
                        size_t sH = 0, const int *active = nullptr);
-// hmap/hseq/seq: also publish hout (kcount + 1 values) to coherent pinned host memory, then
-// seq to *hseq (instance b sHmap entries further on in both); z is only read when vout is; xcl/pos (FP32, single instance): also xcl[pos[i]] = vout[i]
+// publishes a column (h1 + h2, kcount values, then the norm) to hmap in coherent pinned host
+// memory, then seq to *hseq (instance b sHmap entries further on in both); with vout, the new
+// vector z / norm; xcl/pos (FP32, single instance): also xcl[pos[i]] = vout[i]
 void launch_finalize(int is_float, int kcount, const double *h1, const double *h2,
-                     const double *Pn, void *z, int n, void *vout, double *hout, hipStream_t s,
+                     const double *Pn, void *z, int n, void *vout, double *hmap,
+                     unsigned long long *hseq, unsigned long long seq, hipStream_t s,
                      int batch = 1, size_t sZ = 0, size_t sV = 0, size_t sHin = 0,
-                     size_t sH = 0, const int *active = nullptr, double *hmap = nullptr,
-                     unsigned long long *hseq = nullptr, unsigned long long seq = 0,
-                     float *xcl = nullptr, const int *pos = nullptr, size_t sHmap = 0);
+                     size_t sHmap = 0, const int *active = nullptr, float *xcl = nullptr,
+                     const int *pos = nullptr);
 #ifndef WB_ARNOLDI1_KB
 #define WB_ARNOLDI1_KB 160
 #endif
@@ -396,9 +397,8 @@ constexpr int ARNOLDI1_MAX_N = 4096;
 constexpr size_t ARNOLDI1_BYTES = WB_ARNOLDI1_KB * 1024;
 bool arnoldi1_fits(int is_float, int kcount, int n);
 void launch_arnoldi1(int is_float, const void *V, size_t ldv, int kcount, const void *z, int n,
-                     void *vout, double *hout, hipStream_t s, double *hmap,
-                     unsigned long long *hseq, unsigned long long seq, float *xcl,
-                     const int *pos);
+                     void *vout, double *hmap, unsigned long long *hseq,
+                     unsigned long long seq, hipStream_t s, float *xcl, const int *pos);
 // x += V y, y (host, kcount entries) taken along as a launch argument
 void launch_axpy_basis(int is_float, const void *V, size_t ldv, int kcount, const double *y,
                        void *x_acc, int x_is_float, int n, hipStream_t s);

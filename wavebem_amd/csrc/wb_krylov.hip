@@ -154,11 +154,11 @@ __global__ __launch_bounds__(KTHREADS) void k_update_dot(const T *__restrict__ V
     }
 }
 
-// hout[k] = h1[k] + h2[k] (k < kcount), hout[kcount] = sqrt(sum Pn); vout = z / hout[kcount].
+// hmap[k] = h1[k] + h2[k] (k < kcount), hmap[kcount] = sqrt(sum Pn); vout = z / hmap[kcount].
 // Every workgroup forms the norm itself, wavefront-parallel and in the same order.
-// With hmap (coherent pinned host memory, instance b at sHmap entries), the column also goes
-// to the host: every thread of workgroup 0 writes its entries and fences at system scope, then
-// thread 0 publishes seq after them, so a host that reads seq (acquire) sees the column.
+// hmap is coherent pinned host memory (instance b at sHmap entries): every thread of
+// workgroup 0 writes its entries and fences at system scope, then thread 0 publishes seq
+// after them, so a host that reads seq (acquire) sees the column.
 // With xcl (single instance), vout is also written to xcl[pos[i]] (FP32).
 template <typename T>
 __global__ __launch_bounds__(KTHREADS) void k_finalize(int kcount, const double *__restrict__ h1,
@@ -167,7 +167,6 @@ __global__ __launch_bounds__(KTHREADS) void k_finalize(int kcount, const double 
                                                        const double *__restrict__ Pn, int nparts,
                                                        const T *__restrict__ z, size_t sZ,
                                                        int n, T *__restrict__ vout, size_t sV,
-                                                       double *__restrict__ hout, size_t sH,
                                                        const int *__restrict__ active,
                                                        double *__restrict__ hmap,
                                                        unsigned long long *__restrict__ hseq,
@@ -184,11 +183,8 @@ __global__ __launch_bounds__(KTHREADS) void k_finalize(int kcount, const double 
     Pn += (size_t)b * nparts;
     z += b * sZ;
     if (vout) vout += b * sV;
-    hout += b * sH;
-    if (hmap) {
-        hmap += b * sHmap;
-        hseq += b * sHmap;
-    }
+    hmap += b * sHmap;
+    hseq += b * sHmap;
     if (threadIdx.x < 64) {
         double s = 0.0;
         for (int p = threadIdx.x; p < nparts; p += 64) s += Pn[p];
@@ -198,21 +194,13 @@ __global__ __launch_bounds__(KTHREADS) void k_finalize(int kcount, const double 
     __syncthreads();
     const double nv = snorm;
     if (blockIdx.x == 0) {
-        for (int k = threadIdx.x; k < kcount; k += KTHREADS) {
-            const double hk = (h1 ? h1[k] : 0.0) + (h2 ? h2[k] : 0.0);
-            hout[k] = hk;
-            if (hmap) hmap[k] = hk;
-        }
-        if (threadIdx.x == 0) {
-            hout[kcount] = nv;
-            if (hmap) hmap[kcount] = nv;
-        }
-        if (hmap) {
-            __threadfence_system();
-            __syncthreads();
-            if (threadIdx.x == 0)
-                __hip_atomic_store(hseq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
+        for (int k = threadIdx.x; k < kcount; k += KTHREADS)
+            hmap[k] = (h1 ? h1[k] : 0.0) + (h2 ? h2[k] : 0.0);
+        if (threadIdx.x == 0) hmap[kcount] = nv;
+        __threadfence_system();
+        __syncthreads();
+        if (threadIdx.x == 0)
+            __hip_atomic_store(hseq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     if (vout) {
         const double inv = nv > 0 ? 1.0 / nv : 0.0;
@@ -239,7 +227,7 @@ constexpr int A1_THREADS = 1024;
 template <typename T>
 __global__ __launch_bounds__(A1_THREADS) void k_arnoldi1(
     const T *__restrict__ V, size_t ldv, int kcount, const T *__restrict__ z, int n,
-    T *__restrict__ vout, double *__restrict__ hout, double *__restrict__ hmap,
+    T *__restrict__ vout, double *__restrict__ hmap,
     unsigned long long *__restrict__ hseq, unsigned long long seq, float *__restrict__ xcl,
     const int *__restrict__ pos)
 {
@@ -281,11 +269,8 @@ __global__ __launch_bounds__(A1_THREADS) void k_arnoldi1(
     double t = 0.0;
     for (int w = 0; w < A1_THREADS / 64; ++w) t += red[w];
     const double nv = sqrt(t);
-    for (int k = tid; k <= kcount; k += A1_THREADS) {
-        const double hk = k < kcount ? h[0][k] + h[1][k] : nv;
-        hout[k] = hk;
-        hmap[k] = hk;
-    }
+    for (int k = tid; k <= kcount; k += A1_THREADS)
+        hmap[k] = k < kcount ? h[0][k] + h[1][k] : nv;
     __threadfence_system();
     __syncthreads();
     if (tid == 0) __hip_atomic_store(hseq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -377,22 +362,22 @@ void launch_update_dot(int is_float, const void *V, size_t ldv, int kcount, void
 }
 
 void launch_finalize(int is_float, int kcount, const double *h1, const double *h2,
-                     const double *Pn, void *z, int n, void *vout, double *hout, hipStream_t s,
-                     int batch, size_t sZ, size_t sV, size_t sHin, size_t sH,
-                     const int *active, double *hmap, unsigned long long *hseq,
-                     unsigned long long seq, float *xcl, const int *pos, size_t sHmap)
+                     const double *Pn, void *z, int n, void *vout, double *hmap,
+                     unsigned long long *hseq, unsigned long long seq, hipStream_t s, int batch,
+                     size_t sZ, size_t sV, size_t sHin, size_t sHmap, const int *active,
+                     float *xcl, const int *pos)
 {
     // without a new vector one workgroup per instance has all there is to do
     const int parts = krylov_partials_blocks(n);
     dim3 grid(vout ? parts : 1, batch);
     if (is_float)
         hipLaunchKernelGGL(k_finalize<float>, grid, dim3(KTHREADS), 0, s, kcount, h1, h2, sHin,
-                           Pn, parts, (const float *)z, sZ, n, (float *)vout, sV, hout, sH,
-                           active, hmap, hseq, seq, xcl, pos, sHmap);
+                           Pn, parts, (const float *)z, sZ, n, (float *)vout, sV, active, hmap,
+                           hseq, seq, xcl, pos, sHmap);
     else
         hipLaunchKernelGGL(k_finalize<double>, grid, dim3(KTHREADS), 0, s, kcount, h1, h2, sHin,
-                           Pn, parts, (const double *)z, sZ, n, (double *)vout, sV, hout, sH,
-                           active, hmap, hseq, seq, (float *)nullptr, pos, sHmap);
+                           Pn, parts, (const double *)z, sZ, n, (double *)vout, sV, active,
+                           hmap, hseq, seq, (float *)nullptr, pos, sHmap);
 }
 
 // Whether an Arnoldi step with kcount basis vectors goes to k_arnoldi1: the basis it reads
@@ -405,18 +390,17 @@ bool arnoldi1_fits(int is_float, int kcount, int n)
 }
 
 void launch_arnoldi1(int is_float, const void *V, size_t ldv, int kcount, const void *z, int n,
-                     void *vout, double *hout, hipStream_t s, double *hmap,
-                     unsigned long long *hseq, unsigned long long seq, float *xcl,
-                     const int *pos)
+                     void *vout, double *hmap, unsigned long long *hseq,
+                     unsigned long long seq, hipStream_t s, float *xcl, const int *pos)
 {
     if (is_float)
         hipLaunchKernelGGL(k_arnoldi1<float>, dim3(1), dim3(A1_THREADS), 0, s, (const float *)V,
-                           ldv, kcount, (const float *)z, n, (float *)vout, hout, hmap, hseq,
-                           seq, xcl, pos);
+                           ldv, kcount, (const float *)z, n, (float *)vout, hmap, hseq, seq,
+                           xcl, pos);
     else
         hipLaunchKernelGGL(k_arnoldi1<double>, dim3(1), dim3(A1_THREADS), 0, s,
                            (const double *)V, ldv, kcount, (const double *)z, n, (double *)vout,
-                           hout, hmap, hseq, seq, (float *)nullptr, pos);
+                           hmap, hseq, seq, (float *)nullptr, pos);
 }
 
 void launch_axpy_basis(int is_float, const void *V, size_t ldv, int kcount, const double *y,
