@@ -391,17 +391,17 @@ void launch_assemble_tiles(int precision, int q_order, int tc, const double *xro
 //                   walk a task side by side, and every new line made all of them wait for
 //                   one L2 miss;
 //   26.9 / 27.7     this form.  Without its stores it takes 22 ms: the 8-column segments left
-//                   the L2 2.3 times over (47.7 GB for 20.4 GB of entries; 34 GB now).
+//                   the L2 2.3 times over (47.7 GB for 20.4 GB of entries; 31.4 GB now).
 // A small mesh gets four times as many wavefronts, each a quarter as long: 0.75 -> 0.19 ms
 // at 2,915 dofs, 0.27 -> 0.08 ms at 1,083.
 // Three wavefronts per SIMD hold everything in registers; at four, a spilled register reloaded
 // between the stores waits for all of them (loads and stores share one in-order counter).
 //
 // LDS, in regions of STRIP_W x 64 doubles: LO[4] by wavefront, UP[5] by gap modulo 5 (the
-// fifth is the last round's), and the G part's own kept UP: 10 x 4 KB, so that four
-// workgroups fill a CU's 160 KB.  Slot p of a region holds row r at (r ^ 2 p ^ 16 parity):
-// the write-out reads 16 columns (two lines of different parity) x 2 rows per half
-// wavefront from distinct banks.
+// fifth is the last round's), and the G part's own kept UP: 10 x 4 KB.  A CU holds three
+// workgroups, by their registers (the LDS would take four).  Slot p of a region holds row r
+// at (r ^ 2 p ^ 16 parity): the write-out reads 16 columns (two lines of different parity)
+// x 2 rows per half wavefront from distinct banks.
 // Every cell is evaluated once per task it touches: once inside a strip, twice on the
 // boundary between two strips or two tasks of one strip.
 constexpr int STRIP_REGION = STRIP_W * TILE_ROWS;  // doubles

@@ -38,9 +38,10 @@ __device__ __forceinline__ double rsqrt_f64(double r2)
 
 // 2/sqrt(r2) with one Newton step y (3 - r2 y^2) from the hardware estimate: relative error
 // (3/2) eps^2, at most 4.1e-15 with the measured eps above (3 operations; the factor 2 goes
-// into the caller's scale, exactly).  For values stored as FP32 hi + bf16 lo (relative
-// rounding 2^-33 = 1.2e-10) this is 30000 times below the storage error; the FP64 stores
-// use rsqrt_f64.
+// into the caller's scale, exactly).  Over 2^20 values of r2 from e^-12 to e^2: at most
+// 4.12e-15, rms 3.03e-16; y + y e / 2 with e = 1 - r2 y^2, an operation more, 4.12e-15 and
+// 2.99e-16.  For values stored as FP32 hi + bf16 lo (relative rounding 2^-33 = 1.2e-10) this
+// is 30000 times below the storage error; the FP64 stores use rsqrt_f64.
 __device__ __forceinline__ double rsqrt2_f64_newton1(double r2)
 {
     const double y = __builtin_amdgcn_rsq(r2);

@@ -56,7 +56,7 @@ constexpr int F64_RPW = 4, F64_WAVES = 4;
 
 // The blocks past those of the n_rows rows (PB each) write the constraint lines, one thread
 // per line; returns whether this is one of them.  (A launch of its own took 4 us and the gap
-// before it: an FP64 step at 2.9k dofs 2.18 -> 2.12 ms, one product at 1,083 dofs 57 -> 54 us.)
+// before it: an FP64 step at 2.9k dofs 2.18 -> 2.12 ms, one product at 1,083 dofs 49 -> 47 us.)
 template <int PB, typename T>
 __device__ __forceinline__ bool lines_block(int n_rows, const ConLines &L,
                                             const T *__restrict__ x, T *__restrict__ y)

@@ -139,6 +139,11 @@ __device__ __forceinline__ void block_sum(double (&v)[K], double (*lds)[K][8],
 // totals of the block partials part[nb][K], broadcast through LDS (out, K values): the PB / K
 // threads of each k add every (PB / K)-th partial, and their sums are added in thread order
 // (the same bits in every block).  A serial sum by K threads took 10 us for 43 partials.
+// Every block reads all n / PR partials, so a launch reads n^2: small beside the rows' own
+// latency up to the sizes that a context can hold.  One compute_potential_gradients, against
+// a thread per row and 256 rows per block: 2.15 -> 1.22 ms at 11k dofs, 4.3 -> 2.4 at 40k,
+// 5.8 -> 3.9 at 59k, 9.1 -> 7.0 at 95k, 11.6 -> 9.4 at 121k (the FP32-IR matrices of 155k
+// fill the card).
 template <int K>
 __device__ __forceinline__ void sum_parts(const double *__restrict__ part, int nb, double *out)
 {
